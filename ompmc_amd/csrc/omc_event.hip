@@ -79,6 +79,10 @@ constexpr int DEFAULT_TURNS = 24;
 #endif
 constexpr int CHARGED_BLOCKS_PER_CU = OMC_CHARGED_BLOCKS_PER_CU;
 constexpr int PHOTON_BLOCKS_PER_CU = OMC_PHOTON_BLOCKS_PER_CU;
+// Wavefronts of them a compute unit holds at once, by their registers: two a
+// SIMD of the charged kernel, three of the photon kernels.
+constexpr int CHARGED_WAVES_PER_CU = 8;
+constexpr int PHOTON_WAVES_PER_CU = 12;
 // LDS a charged-kernel workgroup may give to the electron bins (12 KB per
 // medium at 150 bins; two workgroups share a CU's 160 KB).  Plans with more
 // media read them from device memory.
@@ -365,6 +369,8 @@ template <class R> void fill_launch(omc_ctx *c, const PhantomDev *pd, EvState<R>
     L.grid_event = o->grid > 0 ? o->grid : cus * PHOTON_BLOCKS_PER_CU;
     L.grid_charged = o->grid > 0 ? o->grid : cus * CHARGED_BLOCKS_PER_CU;
     L.grid_source = cus * 4;
+    L.waves_event = std::min(cus * PHOTON_WAVES_PER_CU, L.grid_event * 4);       // four waves a workgroup
+    L.waves_charged = std::min(cus * CHARGED_WAVES_PER_CU, L.grid_charged * 4);
     L.src.t = L.t;
     L.src.g = L.g;
     L.src.seed = o->seed;

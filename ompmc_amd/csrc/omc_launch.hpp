@@ -42,6 +42,7 @@ template <class R> struct EvLaunch {
     int tlist;                   // deposit-list entries per charged-kernel lane in LDS (0: direct atomics)
     SrcArgs<R> src;              // source of the job (ctl and out are set per round)
     int grid_event, grid_charged, grid_source;   // workgroups: photon kernels, charged kernel, source
+    int waves_event, waves_charged;              // wavefronts of the first two that are resident at once
 };
 
 // Enqueues rounds r0 .. r0+nround-1 of the job whose control block is L.ctl.
