@@ -106,6 +106,18 @@ template <class R> struct alignas(16) MsBin {
 static_assert(sizeof(MsBin<float>) == 16 && sizeof(MsBin<double>) == 32 && offsetof(MsBin<double>, f) == 16,
               "the bin loads below assume this layout");
 
+// Address spaces of the data the kernels read.  The descriptors (Tables, Geom)
+// do not change while a kernel runs: read as constants, a field is one scalar
+// load that the compiler may keep across the tally's stores and atomics.  Read
+// as plain memory it was a vector load again at every use, since any store
+// might have changed it, and each table lookup waited for two loads, its
+// pointer's and its own.
+#define OMC_GLOBAL __attribute__((address_space(1)))
+#define OMC_CONST __attribute__((address_space(4)))
+template <class T> __device__ __forceinline__ const OMC_CONST T &constant(const T *p) {
+    return *(const OMC_CONST T *)p;
+}
+
 // Loads through pointers into device tables and phantom arrays, which live
 // in global memory: addressed as such they compile to global loads instead
 // of flat accesses.
@@ -373,8 +385,8 @@ struct Counters {
 // device memory when they are not staged -- with generic loads; otherwise
 // every bin comes from Tables::cbin with global loads.
 template <class R, class G, class T, bool LDS = false> struct Engine {
-    const Tables<R> &t;
-    const Geom<R> &g;
+    const OMC_CONST Tables<R> &t;
+    const OMC_CONST Geom<R> &g;
     G &rng;
     T &tally;
     Counters cnt;
@@ -386,6 +398,10 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     int aborted = 0;
     int abort_site = 0;
     const CBin<R> *eb = nullptr;    // LDS engines: electron bins (LDS or device memory, same layout)
+
+    // constants of a medium that may differ from lane to lane
+    using MedRef = const OMC_GLOBAL Med<R> &;
+    __device__ __forceinline__ MedRef med_of(int imed) const { return ((const OMC_GLOBAL Med<R> *)t.med)[imed]; }
 
     // the interleaved coefficients of bin l of species qel (0 electrons,
     // 1 positrons) in medium imed, and loads of their fields
@@ -442,7 +458,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // (measured: one photon in ~6e7 FP32 histories, whose garbage Rayleigh
     // fraction then kept it scattering until a guard dropped it).  In FP64
     // the formula stays at 0 there, so the clamp changes nothing.
-    static __device__ __forceinline__ int photon_interval(R gle, const Med<R> &m) {
+    template <class MR> static __device__ __forceinline__ int photon_interval(R gle, const MR &m) {
         const int i = pwlf_i(gle, m.ge1, m.ge0) - 1;
         return i < 0 ? 0 : i;
     }
@@ -599,11 +615,11 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
             do {
                 r0 = rnd();
                 r0 *= pmax;
-                int ib = t.ray_iarr[0] - 1;
-                if ((t.ray_iarr[1] - 1) > ib)
-                    while (r0 >= t.ray_fcum[ib + 1]) ib++;
-                r0 = (r0 - t.ray_fcum[ib]) * t.ray_c[ib];
-                xv = t.ray_xgrid[ib] * M<R>::exp(M<R>::log((R)1.0 + r0) * t.ray_b[ib]);
+                int ib = gld(t.ray_iarr) - 1;
+                if ((gld(t.ray_iarr + 1) - 1) > ib)
+                    while (r0 >= gld(t.ray_fcum + ib + 1)) ib++;
+                r0 = (r0 - gld(t.ray_fcum + ib)) * gld(t.ray_c + ib);
+                xv = gld(t.ray_xgrid + ib) * M<R>::exp(M<R>::log((R)1.0 + r0) * gld(t.ray_b + ib));
             } while ((xv >= xmax) && !stuck(trials_in));
             xv /= eig;
             costhe = (R)1.0 - (R)0.000307444456 * (xv * xv);
@@ -614,7 +630,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         uphi21(p, q, costhe, sinthe);
     }
 
-    __device__ __forceinline__ R pair_rej(const Med<R> &m, R xi, R esedei, R eseder, R tteig) {
+    __device__ __forceinline__ R pair_rej(MedRef m, R xi, R esedei, R eseder, R tteig) {
         R a = (R)1.0 + eseder, b = (R)1.0 + esedei;
         R c = a * b / ((R)2.0 * tteig);
         R xm = xi - (R)0.5;
@@ -625,7 +641,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
 
     // pair production (src/ompmc.c:1447-1685)
     __device__ OMC_INL void pair(int imed, Part<R> &p0, Part<R> &p1) {
-        const Med<R> &m = t.med[imed];
+        MedRef m = med_of(imed);
         const R RM = (R)0.5109989461;
         R eig = p0.e, ese1, ese2;
         int iq1, iq2, l, l1;
@@ -849,7 +865,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         for (;;) {
             R tstep;
             if (imed != -1) {
-                const Med<R> &m = t.med[imed];
+                MedRef m = med_of(imed);
                 lgle = photon_interval(gle, m);
                 R gmfpr0 = pwlf(t.gmfp + (imed * MXGE + lgle), gle);
                 gmfp = gmfpr0 / rhof_of(p);
@@ -917,12 +933,12 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     __device__ __forceinline__ int locate(const R *b, int n, R x, R inv) const {
         int i;
         if (g.uniform) {
-            i = (int)((x - b[0]) * inv);
+            i = (int)((x - gld(b)) * inv);
         } else {
             int lo = 0, hi = n;
             while (hi - lo > 1) {
                 int mid = (lo + hi) >> 1;
-                if (b[mid] <= x) lo = mid;
+                if (gld(b + mid) <= x) lo = mid;
                 else hi = mid;
             }
             i = lo;
@@ -962,7 +978,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
 #pragma unroll
         for (int m = 0; m < MXMED; m++) {
             const int mc = m < t.nmed ? m : 0;
-            const Med<R> &md = t.med[mc];
+            const OMC_CONST Med<R> &md = constant(t.med + mc);
             const int lg = photon_interval(gle, md);
             const R mr = (R)1.0 / (pwlf(t.gmfp + (mc * MXGE + lg), gle) * pwlf(t.cohe + (mc * MXGE + lg), gle));
             const R rm = g.rhof_max[m];
@@ -1018,7 +1034,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         // interacts does so together, once per flight (inside the loop the
         // wave ran the interaction code once per trial in which any lane
         // accepted).  Each lane's operations and draws are the same.
-        const Med<R> &md = t.med[imed];
+        MedRef md = med_of(imed);
         int lgle = photon_interval(gle, md);
         R cohfac = pwlf(t.cohe + (imed * MXGE + lgle), gle);
         return interact(p, q, imed, eig, gle, lgle, cohfac);
@@ -1033,7 +1049,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
 #pragma unroll
         for (int m = 0; m < MXMED; m++) {
             const int mc = m < t.nmed ? m : 0;
-            const Med<R> &md = t.med[mc];
+            const OMC_CONST Med<R> &md = constant(t.med + mc);
             const int lg = photon_interval(gle, md);
             xs.lgle[m] = lg;
             xs.gmfp0[m] = pwlf(t.gmfp + (mc * MXGE + lg), gle);
@@ -1402,7 +1418,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // two-substep multiple scattering, PRESTA-II style (src/ompmc.c:3805-3994)
     __device__ OMC_INL R msdist(const Part<R> &p, int imed, int iq, R rhof, R de, R tustep, R eke, Part<R> &out) {
         const R RM = (R)0.5109989461;
-        const Med<R> &m = t.med[imed];
+        MedRef m = med_of(imed);
         int qel = (1 + iq) / 2;
         Mscats ms = {0, 0, (R)0};
         Spinr sr = {0, 0};
@@ -1514,7 +1530,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // of the energy bin already loaded
     __device__ OMC_INL R eloss(int imed, int iq, R rhof, R tustep, R range, R eke, R elke, int lelke,
                                const PW<R> &q_lo, R rep_lo) {
-        const Med<R> &m = t.med[imed];
+        MedRef m = med_of(imed);
         int qel = (1 + iq) / 2;
         const R *rep = t.range_ep + ((size_t)qel * t.nmed + imed) * MXEKE;
         const PW<R> *dx = iq < 0 ? t.ededx : t.pdedx;
@@ -1587,7 +1603,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     __device__ OMC_INL void brems(Part<R> &pe, Part<R> &pg) {
         const R RM = (R)0.5109989461;
         int imed = medium(pe);
-        const Med<R> &m = t.med[imed];
+        MedRef m = med_of(imed);
         R eie = pe.e;
         int l = eie < (R)50.0 ? 1 : 3, l1 = l + 1;
         R ekin = eie - RM, brmin = m.ap / ekin, waux = -M<R>::log(brmin);
@@ -1672,7 +1688,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // Moller (src/ompmc.c:4377-4453); nothing happens at or below 2*TE (quirk Q4)
     __device__ OMC_INL int moller(Part<R> &p0, Part<R> &p1) {
         const R RM = (R)0.5109989461;
-        const Med<R> &m = t.med[medium(p0)];
+        MedRef m = med_of(medium(p0));
         R eie = p0.e, ekin = eie - RM;
         if (ekin <= (R)2.0 * m.te) return 0;
         R t0 = ekin / RM, e0 = t0 + (R)1.0, extrae = eie - m.thmoll;
@@ -1703,7 +1719,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // Bhabha (src/ompmc.c:4456-4543)
     __device__ OMC_INL void bhabha(Part<R> &p0, Part<R> &p1) {
         const R RM = (R)0.5109989461;
-        const Med<R> &m = t.med[medium(p0)];
+        MedRef m = med_of(medium(p0));
         R eip = p0.e, ekin = eip - RM, t0 = ekin / RM, e0 = t0 + (R)1.0;
         R yy = (R)1.0 / (t0 + (R)2.0);
         R beta2 = (e0 * e0 - (R)1.0) / (e0 * e0);
@@ -1852,7 +1868,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         int lelke = 0;
         if (resume) {
             elke = M<R>::log(eie - RM);
-            lelke = pwlf_i(elke, t.med[imed].eke1, t.med[imed].eke0) - 1;
+            lelke = pwlf_i(elke, med_of(imed).eke1, med_of(imed).eke0) - 1;
         }
         R sigratio = (R)0, rfict = (R)0;
         bool first = true;
@@ -1887,7 +1903,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 sig0 = es.sig0;
                 resume = false;
             } else if (imed != -1) {
-                const Med<R> &m = t.med[imed];
+                MedRef m = med_of(imed);
                 R rn = rnd();
                 if (rn == (R)0.0) rn = (R)1.0E-30;
                 demfp = M<R>::fmax(-M<R>::log(rn), (R)1.0E-5);
@@ -1912,7 +1928,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     tustep = ustep;
                     call_howfar = true;
                 } else {
-                    const Med<R> &m = t.med[imed];
+                    MedRef m = med_of(imed);
                     const R *rep = t.range_ep + ((size_t)qel * t.nmed + imed) * MXEKE;
                     // this step's table entries at (medium, energy bin), loaded
                     // together ahead of the branches below, whose outcome they
@@ -2043,7 +2059,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 if (!called_msdist) {
                     R costhe = (R)1.0, sinthe = (R)0.0;
                     if (do_single) {
-                        const Med<R> &m = t.med[imed];
+                        MedRef m = med_of(imed);
                         R ekems = M<R>::fmax(ekef, g.ecut[imed] - RM);
                         R p2 = ekems * (ekems + (R)2.0 * RM);
                         R beta2 = p2 / (p2 + RM * RM);
@@ -2072,7 +2088,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 if (mv == 0 && eie <= ecut_of(imed)) return electron_stop(p, q, iq, eie, false);
                 medold = imed;
                 if (imed != -1) {
-                    const Med<R> &m = t.med[imed];
+                    MedRef m = med_of(imed);
                     eke = eie - RM;
                     elke = M<R>::log(eke);
                     lelke = pwlf_i(elke, m.eke1, m.eke0) - 1;
@@ -2117,7 +2133,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 brems(p, q);
                 return 1;
             }
-            if (p.e <= t.med[imed].thmoll) {
+            if (p.e <= med_of(imed).thmoll) {
                 if (ebr1 <= (R)0) return 0;
                 brems(p, q);
                 return 1;

@@ -415,7 +415,7 @@ k_event(EvArgs<R> a) {
         bool done = false;
         uint32_t qpos = 0;
         if (have) {
-            Engine<R, StreamAt, Tally, !PHOTON && sizeof(R) == 4> e{*a.t, *a.g, rng, tally,
+            Engine<R, StreamAt, Tally, !PHOTON && sizeof(R) == 4> e{constant(a.t), constant(a.g), rng, tally,
                                                                           {0, 0, 0, 0, 0, 0, 0}, COUNT};
             e.nsplit = a.nsplit;          // roulette of the photons that charged particles produce
             e.eb = eb;
@@ -514,7 +514,7 @@ k_event_split(EvArgs<R> a) {
             tally.init(a.endep + (size_t)slot * a.slot_stride,
                        a.touched ? a.touched + (size_t)slot * a.touch_stride : nullptr);
         }
-        Engine<R, StreamAt, TallyAtomic> e{*a.t, *a.g, rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
+        Engine<R, StreamAt, TallyAtomic> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
         e.nsplit = ns;
         // set-up of the split (src/ompmc.c:1900-1940)
         bool live = have, surv = false;
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(256) k_source(SrcArgs<R> a) {
         StreamAt rng;
         rng.at(a.seed, stream, 0, nullptr);
         TallyNone tn;
-        Engine<R, StreamAt, TallyNone> e{*a.t, *a.g, rng, tn, {0, 0, 0, 0, 0, 0, 0}, false};
+        Engine<R, StreamAt, TallyNone> e{constant(a.t), constant(a.g), rng, tn, {0, 0, 0, 0, 0, 0, 0}, false};
         Part<R> p;
         if (a.use_beamlets) init_history(e, a.bix, beamlet, p);
         else init_history(e, a.dos, p);

@@ -35,12 +35,12 @@ template <class R, class E> __device__ __forceinline__ R sample_energy(E &e, int
     if (!spectrum) return energy;
     R r1 = e.rnd(), r2 = e.rnd();
     int k = (int)M<R>::fmin(deltak * r1, deltak - (R)1.0);
-    return c1[k] + r2 * c2[k];
+    return gld(c1 + k) + r2 * gld(c2 + k);
 }
 
 template <class R, class E> __device__ void init_history(E &e, const SrcDosxyz<R> &s, Part<R> &p) {
     const R RM = (R)0.5109989461;
-    const Geom<R> &g = e.g;
+    const OMC_CONST Geom<R> &g = e.g;
     p.iq = s.charge;
     R ein = sample_energy<R>(e, s.spectrum, s.energy, s.deltak, s.cdfinv1, s.cdfinv2);
     p.e = p.iq != 0 ? ein + RM : ein;
@@ -64,7 +64,7 @@ template <class R, class E> __device__ void init_history(E &e, const SrcDosxyz<R
             fw = p.w * p.w * p.w;
         } while (r3 >= fw && !e.stuck(trials));
     }
-    p.z = g.zb[0];
+    p.z = gld(g.zb);
     p.u = p.x / rxyz;
     p.v = p.y / rxyz;
     int ix, iy;
@@ -72,13 +72,13 @@ template <class R, class E> __device__ void init_history(E &e, const SrcDosxyz<R
         ix = s.ixinl;
     } else {
         ix = s.ixinl - 1;
-        while (ix < g.nx - 1 && g.xb[ix + 1] < p.x) ix++;
+        while (ix < g.nx - 1 && gld(g.xb + ix + 1) < p.x) ix++;
     }
     if (s.ysize == (R)0.0) {
         iy = s.iyinl;
     } else {
         iy = s.iyinl - 1;
-        while (iy < g.ny - 1 && g.yb[iy + 1] < p.y) iy++;
+        while (iy < g.ny - 1 && gld(g.yb + iy + 1) < p.y) iy++;
     }
     p.ix = ix; p.iy = iy; p.iz = 0;
     p.wt = (R)1.0;
@@ -93,14 +93,14 @@ template <class R> __device__ __forceinline__ int entry_index(const R *b, int n,
     int lo = 0, hi = n - 1;            // the answer lies in [lo, hi]
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (b[mid] < x) lo = mid;      // b[1..mid] are all below x (b increases)
+        if (gld(b + mid) < x) lo = mid;      // b[1..mid] are all below x (b increases)
         else hi = mid - 1;
     }
     return lo;
 }
 
 template <class R, class E> __device__ void init_history(E &e, const SrcBeamlets<R> &s, int ib, Part<R> &p) {
-    const Geom<R> &g = e.g;
+    const OMC_CONST Geom<R> &g = e.g;
     const R tiny = sizeof(R) == 8 ? (R)(2.0 * 2.2250738585072014e-308) : (R)0;
     p.iq = 0;
     p.e = sample_energy<R>(e, s.spectrum, s.energy, s.deltak, s.cdfinv1, s.cdfinv2);
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(256) k_history(HistArgs<R> a) {
             TallyAtomic tally;
             tally.init(a.endep + (size_t)slot * a.slot_stride,
                        a.touched ? a.touched + (size_t)slot * a.touch_stride : nullptr);
-            Engine<R, G, TallyAtomic> e{*a.t, *a.g, rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
+            Engine<R, G, TallyAtomic> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
             Part<R> p, q;
             if (a.use_beamlets) init_history(e, a.bix, beamlet, p);
             else init_history(e, a.dos, p);
@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(256) k_history_split(HistArgs<R> a) {
             TallyAtomic tally;
             tally.init(a.endep + (size_t)slot * a.slot_stride,
                        a.touched ? a.touched + (size_t)slot * a.touch_stride : nullptr);
-            Engine<R, G, TallyAtomic> e{*a.t, *a.g, rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
+            Engine<R, G, TallyAtomic> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
             e.nsplit = a.nsplit;
             if (a.use_beamlets) init_history(e, a.bix, beamlet, st[0]);
             else init_history(e, a.dos, st[0]);
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(64) k_sampler(SampArgs<R> a) {
     rng.base = a.rn; rng.pos = a.rn_off[c]; rng.end = a.rn_off[c + 1]; rng.err = a.err;
     TallyRec tally;
     tally.buf = out + 64; tally.cap = (a.out_stride - 64) / 2; tally.n = 0;
-    Engine<R, Replay, TallyRec> e{*a.t, *a.g, rng, tally, {0, 0, 0, 0, 0, 0, 0}, true};
+    Engine<R, Replay, TallyRec> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, true};
     Part<R> p, q;
     int kind = a.kind[c];
     int d = 0;
