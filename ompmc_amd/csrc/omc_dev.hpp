@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace omc {
 
@@ -113,6 +114,7 @@ static_assert(sizeof(MsBin<float>) == 16 && sizeof(MsBin<double>) == 32 && offse
 // might have changed it, and each table lookup waited for two loads, its
 // pointer's and its own.
 #define OMC_GLOBAL __attribute__((address_space(1)))
+#define OMC_LDS __attribute__((address_space(3)))
 #define OMC_CONST __attribute__((address_space(4)))
 template <class T> __device__ __forceinline__ const OMC_CONST T &constant(const T *p) {
     return *(const OMC_CONST T *)p;
@@ -150,9 +152,10 @@ template <class R> __device__ __forceinline__ PW<R> gld(const PW<R> *p) {
 // Tables::cbin holds them as [2][nmed][cb_stride] (electrons, positrons;
 // cb_stride = the largest MEKE + 1); the per-quantity arrays stay for reads
 // at other bins (the range walk of eloss, the end of a step's interval).
-template <class R> struct CBin {
-    PW<R> dedx, sig, tmxs, eta, blcc, q1c, q2c, br1, br2;  // br1/br2: ebr1 (electrons), pbr1/pbr2 (positrons)
+// The fields of a step come first, those of one 16-byte read side by side.
+template <class R> struct alignas(16) CBin {
     R e_lo, range;                                          // e_array and range_ep at the bin
+    PW<R> dedx, tmxs, eta, blcc, sig, q1c, q2c, br1, br2;  // br1/br2: ebr1 (electrons), pbr1/pbr2 (positrons)
 };
 static_assert(sizeof(CBin<float>) % 16 == 0 && sizeof(CBin<double>) % 16 == 0, "copied in 16-byte words");
 
@@ -379,12 +382,26 @@ struct Counters {
     unsigned long long nhowfar, nhownear, ncross, ndep, nrn, nphoton, nelectron;
 };
 
+// ------------------------------------------------------------------ staged data
+// What the workgroups of an event kernel copy to LDS before their loop (ST of
+// the engine): the voxel planes and the media's constants with their cut-offs,
+// and the electron bins of every medium.  A charged particle's step reads
+// the six planes of its voxel, a few constants of its medium and one or more
+// bins, each a different address per lane: from device memory each such round
+// is a gather through the vector cache, the next one waits for it, and at two
+// waves per SIMD little else runs meanwhile.
+constexpr int ST_GEOM = 1, ST_BINS = 2;
+template <class R> struct Staged {
+    const OMC_LDS CBin<R> *bins;            // [nmed][cb_stride], electrons
+    const OMC_LDS Med<R> *med;              // [nmed]
+    const OMC_LDS R *ecut;                  // [MXMED]
+    const OMC_LDS R *xb, *yb, *zb;
+};
+
 // ------------------------------------------------------------------ transport engine
-// LDS: the charged-particle event kernel's engine, whose electron bins are
-// read through `eb` -- the kernel's LDS copy of them, or their place in
-// device memory when they are not staged -- with generic loads; otherwise
-// every bin comes from Tables::cbin with global loads.
-template <class R, class G, class T, bool LDS = false> struct Engine {
+// ST: which tables the kernel has staged in LDS (Staged); the others come from
+// device memory with global loads.
+template <class R, class G, class T, int ST = 0> struct Engine {
     const OMC_CONST Tables<R> &t;
     const OMC_CONST Geom<R> &g;
     G &rng;
@@ -397,30 +414,50 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
     // source line of the loop in abort_site)
     int aborted = 0;
     int abort_site = 0;
-    const CBin<R> *eb = nullptr;    // LDS engines: electron bins (LDS or device memory, same layout)
+    Staged<R> lds = {};             // the staged tables (ST)
 
     // constants of a medium that may differ from lane to lane
-    using MedRef = const OMC_GLOBAL Med<R> &;
-    __device__ __forceinline__ MedRef med_of(int imed) const { return ((const OMC_GLOBAL Med<R> *)t.med)[imed]; }
+    using MedRef = typename std::conditional<(ST & ST_GEOM) != 0, const OMC_LDS Med<R>, const OMC_GLOBAL Med<R>>::type &;
+    __device__ __forceinline__ MedRef med_of(int imed) const {
+        if constexpr ((ST & ST_GEOM) != 0) return lds.med[imed];
+        else return ((const OMC_GLOBAL Med<R> *)t.med)[imed];
+    }
 
-    // the interleaved coefficients of bin l of species qel (0 electrons,
-    // 1 positrons) in medium imed, and loads of their fields
-    __device__ __forceinline__ const CBin<R> *cbin(int qel, int imed, int l) const {
-        // bins past MEKE are never reached below the tables' upper energy;
-        // the clamp keeps a stray index inside the array
-        l = min(max(l, 0), t.cb_stride - 1);
-        if (LDS && qel == 0) return eb + (imed * t.cb_stride + l);
-        return t.cbin + (((size_t)qel * t.nmed + imed) * t.cb_stride + l);
+    // bin l of species qel (0 electrons, 1 positrons) in medium imed.  Bins past
+    // MEKE are never reached below the tables' upper energy; the clamp keeps
+    // a stray index inside the array.
+    __device__ __forceinline__ int bin_at(int imed, int l) const {
+        return imed * t.cb_stride + min(max(l, 0), t.cb_stride - 1);
     }
-    __device__ __forceinline__ PW<R> cld(const PW<R> *p) const {
-        if (LDS) return *p;
-        return gld(p);
+    template <class B> static __device__ __forceinline__ PW<R> bin_pw(const B &q) { return PW<R>{q.c1, q.c0}; }
+    template <class B> static __device__ __forceinline__ void bin_get(const B &b, CBin<R> &o) {
+        o.e_lo = b.e_lo; o.range = b.range;
+        o.dedx = bin_pw(b.dedx); o.tmxs = bin_pw(b.tmxs); o.eta = bin_pw(b.eta); o.blcc = bin_pw(b.blcc);
+        o.sig = bin_pw(b.sig); o.q1c = bin_pw(b.q1c); o.q2c = bin_pw(b.q2c);
+        o.br1 = bin_pw(b.br1); o.br2 = bin_pw(b.br2);
     }
-    __device__ __forceinline__ R cld(const R *p) const {
-        if (LDS) return *p;
-        return gld(p);
+    // (the loads of fields that the caller does not use fall away)
+    __device__ __forceinline__ CBin<R> bin(int qel, int imed, int l) const {
+        const int at = bin_at(imed, l);
+        CBin<R> b;
+        if constexpr ((ST & ST_BINS) != 0) {
+            bin_get(lds.bins[at], b);
+            if (qel != 0) bin_get(((const OMC_GLOBAL CBin<R> *)t.cbin)[t.nmed * t.cb_stride + at], b);
+        } else {
+            bin_get(((const OMC_GLOBAL CBin<R> *)t.cbin)[qel * t.nmed * t.cb_stride + at], b);
+        }
+        return b;
     }
-    __device__ __forceinline__ R cpw(const PW<R> *p, R lv) const { return pwlf(cld(p), lv); }
+    // range at the lower edge of bin l, and that edge, at bins other than the
+    // particle's own
+    __device__ __forceinline__ R range_at(int qel, int imed, int l) const {
+        if constexpr ((ST & ST_BINS) != 0) return bin(qel, imed, l).range;
+        return gld(t.range_ep + ((size_t)qel * t.nmed + imed) * MXEKE + l);
+    }
+    __device__ __forceinline__ R e_at(int qel, int imed, int l) const {
+        if constexpr ((ST & ST_BINS) != 0) return bin(qel, imed, l).e_lo;
+        return gld(t.e_array + (imed * MXEKE + l));
+    }
     double esc = 0.0;               // wt * E of photons that left the phantom (energy balance)
     double lost = 0.0;              // energy dropped without a deposit (energy balance)
 
@@ -480,7 +517,11 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         return p.ix < 0 ? (R)0 : gld(g.rhof + (p.ix + g.nx * (p.iy + g.ny * p.iz)));
     }
     __device__ __forceinline__ R pcut_of(int imed) const { return imed < 0 ? (R)0 : g.pcut[imed]; }
-    __device__ __forceinline__ R ecut_of(int imed) const { return imed < 0 ? (R)0 : g.ecut[imed]; }
+    __device__ __forceinline__ R ecut_at(int imed) const {
+        if constexpr ((ST & ST_GEOM) != 0) return lds.ecut[imed];
+        return g.ecut[imed];
+    }
+    __device__ __forceinline__ R ecut_of(int imed) const { return imed < 0 ? (R)0 : ecut_at(imed); }
 
     // ausgab (omc_dosxyz.c:683-694)
     __device__ __forceinline__ void ausgab(const Part<R> &p, R edep) {
@@ -488,58 +529,74 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
         tally.add(region(p), (double)(p.wt * edep));
     }
 
-    // howfar (omc_dosxyz.c:187-297): distance to the next voxel plane along z,
-    // then x, then y with strict '<' (ties go to the first axis tested).
-    // Returns the move: 0 none, +-1 x, +-2 y, +-3 z; *leaves when the new
-    // region is outside.  The caller has checked p.ix >= 0.
-    __device__ __forceinline__ int howfar(const Part<R> &p, R &ustep, bool &leaves) {
-        if (count) cnt.nhowfar++;
-        int mv = 0;
-        R dist;
-        leaves = false;
-        if (p.w > (R)0) {
-            dist = (gld(g.zb + (p.iz + 1)) - p.z) / p.w;
-            if (dist < ustep) { ustep = dist; mv = 3; leaves = p.iz == g.nz - 1; }
-        } else if (p.w < (R)0) {
-            dist = -(p.z - gld(g.zb + (p.iz))) / p.w;
-            if (dist < ustep) { ustep = dist; mv = -3; leaves = p.iz == 0; }
-        }
-        if (p.u > (R)0) {
-            dist = (gld(g.xb + (p.ix + 1)) - p.x) / p.u;
-            if (dist < ustep) { ustep = dist; mv = 1; leaves = p.ix == g.nx - 1; }
-        } else if (p.u < (R)0) {
-            dist = -(p.x - gld(g.xb + (p.ix))) / p.u;
-            if (dist < ustep) { ustep = dist; mv = -1; leaves = p.ix == 0; }
-        }
-        if (p.v > (R)0) {
-            dist = (gld(g.yb + (p.iy + 1)) - p.y) / p.v;
-            if (dist < ustep) { ustep = dist; mv = 2; leaves = p.iy == g.ny - 1; }
-        } else if (p.v < (R)0) {
-            dist = -(p.y - gld(g.yb + (p.iy))) / p.v;
-            if (dist < ustep) { ustep = dist; mv = -2; leaves = p.iy == 0; }
-        }
-        return mv;
+    // voxel planes: from LDS where they are staged
+    __device__ __forceinline__ R plane_x(int i) const {
+        if constexpr ((ST & ST_GEOM) != 0) return lds.xb[i];
+        return gld(g.xb + i);
+    }
+    __device__ __forceinline__ R plane_y(int i) const {
+        if constexpr ((ST & ST_GEOM) != 0) return lds.yb[i];
+        return gld(g.yb + i);
+    }
+    __device__ __forceinline__ R plane_z(int i) const {
+        if constexpr ((ST & ST_GEOM) != 0) return lds.zb[i];
+        return gld(g.zb + i);
+    }
+    // the six planes of the particle's voxel, loaded together (p.ix >= 0)
+    struct Planes { R x0, x1, y0, y1, z0, z1; };
+    __device__ __forceinline__ void planes(const Part<R> &p, Planes &b) const {
+        b.x0 = plane_x(p.ix); b.x1 = plane_x(p.ix + 1);
+        b.y0 = plane_y(p.iy); b.y1 = plane_y(p.iy + 1);
+        b.z0 = plane_z(p.iz); b.z1 = plane_z(p.iz + 1);
     }
 
-    __device__ __forceinline__ void apply_move(Part<R> &p, int mv, bool leaves) {
+    // howfar (omc_dosxyz.c:187-297): distance to the next voxel plane along z,
+    // then x, then y with strict '<' (ties go to the first axis tested), from
+    // the planes ahead of the particle.  Returns the move: 0 none, +-1 x, +-2 y,
+    // +-3 z.  The caller has checked p.ix >= 0.
+    __device__ __forceinline__ int howfar(const Part<R> &p, R px, R py, R pz, R &ustep) {
+        if (count) cnt.nhowfar++;
+        int mv = 0;
+        R dist = (pz - p.z) / p.w;
+        if (p.w != (R)0 && dist < ustep) { ustep = dist; mv = p.w > (R)0 ? 3 : -3; }
+        dist = (px - p.x) / p.u;
+        if (p.u != (R)0 && dist < ustep) { ustep = dist; mv = p.u > (R)0 ? 1 : -1; }
+        dist = (py - p.y) / p.v;
+        if (p.v != (R)0 && dist < ustep) { ustep = dist; mv = p.v > (R)0 ? 2 : -2; }
+        return mv;
+    }
+    __device__ __forceinline__ int howfar(const Part<R> &p, const Planes &b, R &ustep) {
+        return howfar(p, p.u > (R)0 ? b.x1 : b.x0, p.v > (R)0 ? b.y1 : b.y0, p.w > (R)0 ? b.z1 : b.z0, ustep);
+    }
+    // the same for a flight that has no use for the other three planes
+    __device__ __forceinline__ int howfar(const Part<R> &p, R &ustep) {
+        return howfar(p, plane_x(p.ix + (p.u > (R)0)), plane_y(p.iy + (p.v > (R)0)), plane_z(p.iz + (p.w > (R)0)),
+                      ustep);
+    }
+
+    // into the next voxel, or out of the phantom
+    __device__ __forceinline__ void apply_move(Part<R> &p, int mv) {
         if (count) cnt.ncross++;
-        if (leaves) { p.ix = -1; return; }
-        if (mv == 1) p.ix++; else if (mv == -1) p.ix--;
-        else if (mv == 2) p.iy++; else if (mv == -2) p.iy--;
-        else if (mv == 3) p.iz++; else if (mv == -3) p.iz--;
+        const int ix = p.ix + (mv == 1) - (mv == -1), iy = p.iy + (mv == 2) - (mv == -2),
+                  iz = p.iz + (mv == 3) - (mv == -3);
+        if ((unsigned)ix >= (unsigned)g.nx || (unsigned)iy >= (unsigned)g.ny || (unsigned)iz >= (unsigned)g.nz) {
+            p.ix = -1;
+            return;
+        }
+        p.ix = ix; p.iy = iy; p.iz = iz;
     }
 
     // hownear (omc_dosxyz.c:299-334)
-    __device__ __forceinline__ R hownear(const Part<R> &p) {
+    __device__ __forceinline__ R hownear(const Part<R> &p, const Planes &b) {
         if (count) cnt.nhownear++;
         if (p.ix < 0) return (R)0;
         R tp = (R)1.0E10;
-        tp = M<R>::fmin(tp, gld(g.xb + (p.ix + 1)) - p.x);
-        tp = M<R>::fmin(tp, p.x - gld(g.xb + (p.ix)));
-        tp = M<R>::fmin(tp, gld(g.yb + (p.iy + 1)) - p.y);
-        tp = M<R>::fmin(tp, p.y - gld(g.yb + (p.iy)));
-        tp = M<R>::fmin(tp, gld(g.zb + (p.iz + 1)) - p.z);
-        tp = M<R>::fmin(tp, p.z - gld(g.zb + (p.iz)));
+        tp = M<R>::fmin(tp, b.x1 - p.x);
+        tp = M<R>::fmin(tp, p.x - b.x0);
+        tp = M<R>::fmin(tp, b.y1 - p.y);
+        tp = M<R>::fmin(tp, p.y - b.y0);
+        tp = M<R>::fmin(tp, b.z1 - p.z);
+        tp = M<R>::fmin(tp, p.z - b.z0);
         return tp;
     }
 
@@ -882,14 +939,13 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 esc += (double)p.wt * (double)eig;
                 return -1;
             }
-            bool leaves;
-            int mv = howfar(p, ustep, leaves);
+            int mv = howfar(p, ustep);
             p.x += ustep * p.u;
             p.y += ustep * p.v;
             p.z += ustep * p.w;
             if (imed != -1) dpmfp = M<R>::fmax((R)0.0, dpmfp - ustep / gmfp);
             if (mv != 0) {
-                apply_move(p, mv, leaves);
+                apply_move(p, mv);
                 imed = medium(p);
             }
             if (imed != -1 && dpmfp <= (R)1.0E-05) break;
@@ -1112,14 +1168,13 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 esc += (double)left * (double)p.wt * (double)p.e;
                 return false;
             }
-            bool leaves;
-            int mv = howfar(p, ustep, leaves);
+            int mv = howfar(p, ustep);
             p.x += ustep * p.u;
             p.y += ustep * p.v;
             p.z += ustep * p.w;
             if (imed != -1) dpmfp = M<R>::fmax((R)0.0, dpmfp - ustep / gmfp);
             if (mv != 0) {
-                apply_move(p, mv, leaves);
+                apply_move(p, mv);
                 voxel_of(p, imed, rho);
             }
             if (imed != -1 && dpmfp <= (R)1.0E-05) return true;
@@ -1440,11 +1495,11 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
             lelke = 0;
             elke = ((R)1.0 - m.eke0) / m.eke1;
         }
-        const CBin<R> *cb = cbin(qel, imed, lelke);
-        R etap = cpw(&cb->eta, elke);
-        R xi_corr = cpw(&cb->q1c, elke);
-        R gamma = cpw(&cb->q2c, elke);
-        R ms_corr = cpw(&cb->blcc, elke);
+        const CBin<R> cb = bin(qel, imed, lelke);
+        R etap = pwlf(cb.eta, elke);
+        R xi_corr = pwlf(cb.q1c, elke);
+        R gamma = pwlf(cb.q2c, elke);
+        R ms_corr = pwlf(cb.blcc, elke);
         chia2 *= etap;
         lambda /= (etap * ((R)1.0 + chia2));
         lambda *= ms_corr;
@@ -1509,7 +1564,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
 
     // CSDA path length inside one PWLF interval (src/ompmc.c:3997-4032)
     __device__ OMC_INL R drange(int imed, int iq, int lelke, R ekei, R ekef, R elkei, R elkef) {
-        return drange(cld(&cbin((1 + iq) / 2, imed, lelke)->dedx), ekei, ekef, elkei, elkef);
+        return drange(bin((1 + iq) / 2, imed, lelke).dedx, ekei, ekef, elkei, elkef);
     }
     // the same with the interval's stopping-power entry already loaded
     __device__ OMC_INL R drange(const PW<R> &q, R ekei, R ekef, R elkei, R elkef) {
@@ -1523,8 +1578,8 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
 
     // sub-threshold energy loss over a path tustep (src/ompmc.c:4034-4126)
     __device__ OMC_INL R eloss(int imed, int iq, R rhof, R tustep, R range, R eke, R elke, int lelke) {
-        const CBin<R> *cb = cbin((1 + iq) / 2, imed, lelke);
-        return eloss(imed, iq, rhof, tustep, range, eke, elke, lelke, cld(&cb->dedx), cld(&cb->range));
+        const CBin<R> cb = bin((1 + iq) / 2, imed, lelke);
+        return eloss(imed, iq, rhof, tustep, range, eke, elke, lelke, cb.dedx, cb.range);
     }
     // the same with the stopping-power entry and the range at the lower edge
     // of the energy bin already loaded
@@ -1532,8 +1587,6 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                                const PW<R> &q_lo, R rep_lo) {
         MedRef m = med_of(imed);
         int qel = (1 + iq) / 2;
-        const R *rep = t.range_ep + ((size_t)qel * t.nmed + imed) * MXEKE;
-        const PW<R> *dx = iq < 0 ? t.ededx : t.pdedx;
         R de, fedep;
         R tuss = range - rep_lo / rhof;
         if (tuss >= tustep) {
@@ -1549,11 +1602,11 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
             if (tuss <= (R)0) {
                 de = eke - m.te * (R)0.99;
             } else {
-                while (l > 0 && tuss < gld(rep + (l))) l -= 1;
+                while (l > 0 && tuss < range_at(qel, imed, l)) l -= 1;
                 R elktmp = ((R)(l + 2) - m.eke0) / m.eke1;
-                R eketmp = gld(t.e_array + (imed * MXEKE + l + 1));
-                tuss = (gld(rep + (l + 1)) - tuss) / rhof;
-                const PW<R> q = gld(dx + (MXEKE * imed + l));
+                R eketmp = e_at(qel, imed, l + 1);
+                tuss = (range_at(qel, imed, l + 1) - tuss) / rhof;
+                const PW<R> q = bin(qel, imed, l).dedx;
                 R dedxmid = pwlf(q, elktmp);
                 R aux = q.c1 / dedxmid;
                 de = dedxmid * tuss * rhof;
@@ -1910,8 +1963,8 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 elke = M<R>::log(eke);
                 lelke = pwlf_i(elke, m.eke1, m.eke0) - 1;
                 if (m.sig_mono[qel]) {
-                    const CBin<R> *cb = cbin(qel, imed, lelke);
-                    sig0 = cpw(&cb->sig, elke) / cpw(&cb->dedx, elke);
+                    const CBin<R> cb = bin(qel, imed, lelke);
+                    sig0 = pwlf(cb.sig, elke) / pwlf(cb.dedx, elke);
                 } else {
                     sig0 = iq < 0 ? m.esig_e : m.psig_e;
                 }
@@ -1922,6 +1975,8 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 PW<R> q_dedx = {(R)0, (R)0};     // stopping power and range at this step's energy bin
                 R rep_lo = (R)0;                 // (loaded below for a step in a medium)
                 Part<R> fin;
+                Planes pl = {};                  // of the voxel, for hownear and howfar
+                if (p.ix >= 0) planes(p, pl);
                 if (imed == -1) {
                     tstep = (R)10.0E8;
                     ustep = tstep;
@@ -1929,17 +1984,14 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     call_howfar = true;
                 } else {
                     MedRef m = med_of(imed);
-                    const R *rep = t.range_ep + ((size_t)qel * t.nmed + imed) * MXEKE;
                     // this step's table entries at (medium, energy bin), loaded
                     // together ahead of the branches below, whose outcome they
                     // do not depend on (same values as loading them where used)
-                    const CBin<R> *cb = cbin(qel, imed, lelke);
-                    q_dedx = cld(&cb->dedx);
-                    const PW<R> q_tmxs = cld(&cb->tmxs);
-                    const PW<R> q_eta = cld(&cb->eta);
-                    const PW<R> q_msc = cld(&cb->blcc);
-                    const R e_lo = cld(&cb->e_lo);
-                    rep_lo = cld(&cb->range);
+                    const CBin<R> cb = bin(qel, imed, lelke);
+                    q_dedx = cb.dedx;
+                    const PW<R> q_tmxs = cb.tmxs, q_eta = cb.eta, q_msc = cb.blcc;
+                    const R e_lo = cb.e_lo;
+                    rep_lo = cb.range;
                     rhof = rhof_voxel;           // the reference reloads the density here, not at the move
                     if (sig0 <= (R)0.0) {
                         tstep = (R)10.0E8;
@@ -1959,10 +2011,10 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                                     R ekei = e_lo;
                                     R elkei = ((R)(lelke + 1) - m.eke0) / m.eke1;
                                     R tuss = drange(q_dedx, eke, ekei, elke, elkei);
-                                    ekei = gld(t.e_array + (imed * MXEKE + lelkef + 1));
+                                    ekei = e_at(qel, imed, lelkef + 1);
                                     elkei = ((R)(lelkef + 2) - m.eke0) / m.eke1;
                                     tstep = drange(imed, iq, lelkef, ekei, ekef, elkei, elkef);
-                                    tstep += tuss + rep_lo - gld(rep + (lelkef + 1));
+                                    tstep += tuss + rep_lo - range_at(qel, imed, lelkef + 1);
                                 }
                             }
                             total_tstep = tstep;
@@ -1980,7 +2032,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     range += rep_lo;
                     range /= rhof;
                     tustep = M<R>::fmin(M<R>::fmin(tstep, tmxs), range);
-                    tperp = hownear(p);
+                    tperp = hownear(p, pl);
                     R blccl = rhof * m.blcc, xccl = rhof * m.xcc;
                     R p2 = eke * (eke + (R)2.0 * RM);
                     R beta2 = p2 / (p2 + RM * RM);
@@ -2020,13 +2072,12 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     }
                 }
                 int mv = 0;
-                bool leaves = false;
                 if (call_howfar) {
                     if (p.ix < 0) {
                         if (count) cnt.nhowfar++;
                         return electron_stop(p, q, iq, eie, true);
                     }
-                    mv = howfar(p, ustep, leaves);
+                    mv = howfar(p, pl, ustep);
                 }
                 if (ustep < (R)0) ustep = (R)0.0;
                 R vstep;
@@ -2038,7 +2089,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                         p.z += p.w * vstep;
                     }
                     if (mv != 0) {
-                        apply_move(p, mv, leaves);
+                        apply_move(p, mv);
                         imed = medium(p);
                         rhof_voxel = rhof_of(p);    // taken into rhof where the reference reloads it
                     }
@@ -2060,14 +2111,16 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     R costhe = (R)1.0, sinthe = (R)0.0;
                     if (do_single) {
                         MedRef m = med_of(imed);
-                        R ekems = M<R>::fmax(ekef, g.ecut[imed] - RM);
+                        R ekems = M<R>::fmax(ekef, ecut_at(imed) - RM);
                         R p2 = ekems * (ekems + (R)2.0 * RM);
                         R beta2 = p2 / (p2 + RM * RM);
                         R chia2 = m.xcc / ((R)4.0 * m.blcc * p2);
                         R elkems = M<R>::log(ekems);
                         int lelkems = pwlf_i(elkems, m.eke1, m.eke0) - 1;
-                        R etap = iq < 0 ? pwlf(t.etae + (MXEKE * imed + lelkems), elkems)
-                                        : pwlf(t.etap + (MXEKE * imed + lelkems), elkems);
+                        PW<R> q_ems;
+                        if constexpr ((ST & ST_BINS) != 0) q_ems = bin(qel, imed, lelkems).eta;
+                        else q_ems = gld((iq < 0 ? t.etae : t.etap) + (MXEKE * imed + lelkems));
+                        R etap = pwlf(q_ems, elkems);
                         chia2 *= etap;
                         sscat(imed, qel, chia2, elkems, beta2, costhe, sinthe);
                     }
@@ -2094,7 +2147,7 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                     lelke = pwlf_i(elke, m.eke1, m.eke0) - 1;
                 }
                 if (mv != 0) {
-                    apply_move(p, mv, leaves);
+                    apply_move(p, mv);
                     imed = medium(p);
                     rhof_voxel = rhof_of(p);    // taken into rhof where the reference reloads it
                 }
@@ -2120,14 +2173,14 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
                 }
             } while (demfp >= (R)1.0E-5);
             if ((imed != medold) || (ustep == (R)0.0) || (imed == -1)) continue;
-            const CBin<R> *cbf = cbin(qel, imed, lelke);
-            R sigf = cpw(&cbf->sig, elke) / cpw(&cbf->dedx, elke);
+            const CBin<R> cbf = bin(qel, imed, lelke);
+            R sigf = pwlf(cbf.sig, elke) / pwlf(cbf.dedx, elke);
             sigratio = sigf / sig0;
             rfict = rnd();
         } while (rfict >= sigratio);
-        const CBin<R> *cbi = cbin(qel, imed, lelke);
+        const CBin<R> cbi = bin(qel, imed, lelke);
         if (iq < 0) {
-            R ebr1 = cpw(&cbi->br1, elke);
+            R ebr1 = pwlf(cbi.br1, elke);
             R rn = rnd();
             if (rn <= ebr1) {
                 brems(p, q);
@@ -2140,13 +2193,13 @@ template <class R, class G, class T, bool LDS = false> struct Engine {
             }
             return moller(p, q);
         }
-        R pbr1 = cpw(&cbi->br1, elke);
+        R pbr1 = pwlf(cbi.br1, elke);
         R rn = rnd();
         if (rn < pbr1) {
             brems(p, q);
             return 1;
         }
-        R pbr2 = cpw(&cbi->br2, elke);
+        R pbr2 = pwlf(cbi.br2, elke);
         if (rn < pbr2) bhabha(p, q);
         else annih(p, q);
         return 1;

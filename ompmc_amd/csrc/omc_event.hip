@@ -87,6 +87,10 @@ constexpr int PHOTON_WAVES_PER_CU = 12;
 // medium at 150 bins; two workgroups share a CU's 160 KB).  Plans with more
 // media read them from device memory.
 constexpr size_t MAX_LDS_TABLES = 64 * 1024;
+// LDS it may give to the media's constants and the voxel planes: 4.2 KB on a
+// 256x256x200 phantom in FP32, 9 KB in FP64.  Phantoms with more planes than
+// this (about 5800 in FP32) read every table from device memory.
+constexpr size_t MAX_LDS_GEOM = 24 * 1024;
 // Entries of a charged-kernel lane's deposit list (TallyList), 16 bytes each
 // for the 256 lanes of a workgroup; the lists are used where bins and lists
 // together leave room for two workgroups per CU.  Eight entries measured the
@@ -218,7 +222,7 @@ int run_job(hipStream_t st, EvState<R> &S, EvLaunch<R> &L, long long nhist, int 
     constexpr int K = 4;
     static_assert(K % 2 == 0, "chunks must start at even rounds");
     bool use_graph = L.graph && !timing;
-    js.lds_bytes = (uint64_t)L.eb_words * 16u;
+    js.lds_bytes = count ? 0 : (uint64_t)L.eb_words * 16u;     // the counting kernels stage nothing
     GraphExec gx;
     // With photon splitting one split puts up to 2 x nsplit charged particles
     // into the queues: a round injects at most target / nsplit primaries, so
@@ -357,13 +361,22 @@ template <class R> void fill_launch(omc_ctx *c, const PhantomDev *pd, EvState<R>
     L.graph = o->graph >= 0 ? 1 : 0;
     {
         const Tables<R> &ht = host_tables_of<R>(c);
+        const omc_phantom &ph = pd->host;
+        const bool fp32 = std::is_same<R, float>::value;
         L.ebin = ht.cbin;
-        const size_t bytes = (size_t)ht.nmed * ht.cb_stride * sizeof(CBin<R>);
-        if (std::is_same<R, float>::value && o->lds_tables >= 0 && bytes <= MAX_LDS_TABLES)
-            L.eb_words = (int)(bytes / 16);
-        // FP32: the deposit lists, where they fit beside the bins in two workgroups per CU
-        if (std::is_same<R, float>::value && (size_t)L.eb_words * 16 + TALLY_LIST_BYTES <= MAX_LDS_PER_GROUP)
-            L.tlist = TALLY_LIST;
+        const size_t bins = (size_t)ht.nmed * ht.cb_stride * sizeof(CBin<R>);
+        const bool stage_bins = fp32 && o->lds_tables >= 0 && bins <= MAX_LDS_TABLES;
+        L.lds_split = lds_layout<R>(ht.nmed, ph.nx, ph.ny, ph.nz, 0, 0);
+        if (L.lds_split.bytes <= (int)MAX_LDS_GEOM) {
+            L.st_split = ST_GEOM;
+            L.st_charged = stage_bins ? ST_GEOM | ST_BINS : ST_GEOM;
+            L.eb_words = stage_bins ? (int)(bins / 16) : 0;
+        }
+        // FP32: the deposit lists, where they fit beside the tables in two workgroups per CU
+        const size_t tables = L.st_charged ? (size_t)L.eb_words * 16 + L.lds_split.bytes : 0;
+        if (fp32 && tables + TALLY_LIST_BYTES <= MAX_LDS_PER_GROUP) L.tlist = TALLY_LIST;
+        L.lds_charged = lds_layout<R>(ht.nmed, ph.nx, ph.ny, ph.nz, (size_t)L.eb_words * 16,
+                                      L.tlist ? TALLY_LIST_BYTES : 0);
     }
     int cus = device_cus(c->device);
     L.grid_event = o->grid > 0 ? o->grid : cus * PHOTON_BLOCKS_PER_CU;

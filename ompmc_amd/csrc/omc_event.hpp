@@ -101,6 +101,21 @@ __device__ __forceinline__ void note_drop(EvCtl *c, int why, int site, const Par
     }
 }
 
+// Dynamic LDS of an event kernel, byte offsets: the electron bins (ST_BINS)
+// from 0, then the media, their cut-offs and the voxel planes (ST_GEOM), then
+// the deposit lists (TallyList).  `bytes` is the whole.
+struct LdsLayout { int med, ecut, planes, list, bytes; };
+template <class R> inline LdsLayout lds_layout(int nmed, int nx, int ny, int nz, size_t bin_bytes, size_t list_bytes) {
+    auto up = [](size_t n) { return (n + 15) / 16 * 16; };
+    LdsLayout l;
+    l.med = (int)up(bin_bytes);
+    l.ecut = l.med + (int)up(sizeof(Med<R>) * nmed);
+    l.planes = l.ecut + (int)up(sizeof(R) * MXMED);
+    l.list = l.planes + (int)up(sizeof(R) * (nx + ny + nz + 3));
+    l.bytes = l.list + (int)list_bytes;
+    return l;
+}
+
 template <class R> struct EvArgs {
     const Tables<R> *t;
     const Geom<R> *g;
@@ -124,8 +139,9 @@ template <class R> struct EvArgs {
     int delta;                        // photons: 1 delta tracking, 0 voxel-by-voxel flight
     int nsplit;                       // photon splitting factor (vrt.nsplit); > 1 runs k_event_split for photons
     EvCtl *ctl;                       // the job's control block (guard reports)
-    const CBin<R> *ebin;              // charged kernel: the electron half of Tables::cbin
-    int eb_words;                     // its size in 16-byte words when copied to LDS (0: read in place)
+    const CBin<R> *ebin;              // ST_BINS kernels: the electron half of Tables::cbin
+    int eb_words;                     // its size in 16-byte words
+    LdsLayout lds;                    // where the staged tables and lists start
     int tlist;                        // charged kernel: deposit-list entries per lane in LDS (TallyList)
     int waves;                        // wavefronts of this launch the device holds at once (lane_share)
 };
@@ -222,6 +238,39 @@ __device__ __forceinline__ void emit(const EvArgs<R> &a, bool want, const Part<R
 // half or twice the wavefronts (1024, 4096) the same to 5%.
 __device__ __forceinline__ int lane_share(long long n, int waves) {
     return n >= 64ll * waves ? 64 : (int)((n + waves - 1) / waves);
+}
+
+// Copies the tables of ST to LDS; every thread of the workgroup calls it.
+template <class R, int ST>
+__device__ __forceinline__ Staged<R> stage(const EvArgs<R> &a, unsigned char *base) {
+    Staged<R> s = {};
+    if constexpr ((ST & ST_BINS) != 0) {
+        uint4 *dst = reinterpret_cast<uint4 *>(base);
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.ebin);
+        for (int i = threadIdx.x; i < a.eb_words; i += blockDim.x) dst[i] = src[i];
+        s.bins = (const OMC_LDS CBin<R> *)base;
+    }
+    if constexpr ((ST & ST_GEOM) != 0) {
+        const OMC_CONST Tables<R> &t = constant(a.t);
+        const OMC_CONST Geom<R> &g = constant(a.g);
+        static_assert(sizeof(Med<R>) % 4 == 0, "copied in words");
+        uint32_t *dm = reinterpret_cast<uint32_t *>(base + a.lds.med);
+        const uint32_t *sm = reinterpret_cast<const uint32_t *>(t.med);
+        for (int i = threadIdx.x; i < t.nmed * (int)(sizeof(Med<R>) / 4); i += blockDim.x) dm[i] = gld(sm + i);
+        R *ec = reinterpret_cast<R *>(base + a.lds.ecut);
+        if (threadIdx.x < MXMED) ec[threadIdx.x] = g.ecut[threadIdx.x];
+        R *xb = reinterpret_cast<R *>(base + a.lds.planes), *yb = xb + g.nx + 1, *zb = yb + g.ny + 1;
+        for (int i = threadIdx.x; i <= g.nx; i += blockDim.x) xb[i] = gld(g.xb + i);
+        for (int i = threadIdx.x; i <= g.ny; i += blockDim.x) yb[i] = gld(g.yb + i);
+        for (int i = threadIdx.x; i <= g.nz; i += blockDim.x) zb[i] = gld(g.zb + i);
+        s.med = (const OMC_LDS Med<R> *)dm;
+        s.ecut = (const OMC_LDS R *)ec;
+        s.xb = (const OMC_LDS R *)xb;
+        s.yb = (const OMC_LDS R *)yb;
+        s.zb = (const OMC_LDS R *)zb;
+    }
+    if constexpr (ST != 0) __syncthreads();
+    return s;
 }
 
 // Charged kernel's tally.  Like TallyAtomic it sums a lane's consecutive
@@ -335,32 +384,21 @@ __device__ __forceinline__ void flush_counters(unsigned long long *dst, const Co
 // travels with the particle (high bits of its phase word): a particle that
 // would make no progress is dropped and reported after a.max_age requeues,
 // instead of cycling through rounds until the job's round guard ends it.
-template <class R, bool PHOTON, bool COUNT>
+template <class R, bool PHOTON, bool COUNT, int ST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PHOTON ? 1 : OMC_CHARGED_WAVES_PER_EU)))
 k_event(EvArgs<R> a) {
     // the charged queue: low band [0, n_lo), then the high band from cap - 1 down
     const unsigned long long pk = *a.n_in;
-    // Charged kernel: the electron bins of every medium (nmed x (MEKE + 1)
-    // records of 80 bytes, at most 64 KiB; launched with that much dynamic
-    // LDS) are copied to LDS once per workgroup, and the step loop reads its
-    // per-bin coefficients there instead of from device memory.
     extern __shared__ __align__(16) unsigned char omc_lds[];
-    const CBin<R> *eb = a.ebin;
-    if (!PHOTON && a.eb_words > 0) {
-        uint4 *dst = reinterpret_cast<uint4 *>(omc_lds);
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.ebin);
-        for (int i = threadIdx.x; i < a.eb_words; i += blockDim.x) dst[i] = src[i];
-        __syncthreads();
-        eb = reinterpret_cast<const CBin<R> *>(omc_lds);
-    }
-    // FP32 charged kernel: each lane's deposit list follows the bins in LDS,
+    const Staged<R> lds = stage<R, ST>(a, omc_lds);
+    // FP32 charged kernel: each lane's deposit list follows the tables in LDS,
     // keys [tlist][blockDim.x] then energies [tlist][blockDim.x].  (The FP64
     // kernel, which spills registers, ran 1% slower with the lists.)
     constexpr bool LIST = !PHOTON && sizeof(R) == 4;
     using Tally = typename std::conditional<LIST, TallyList, TallyAtomic>::type;
     Tally tally;
     if constexpr (LIST) {
-        unsigned char *lst = omc_lds + (size_t)a.eb_words * 16u;
+        unsigned char *lst = omc_lds + a.lds.list;
         tally.key = reinterpret_cast<int2 *>(lst) + threadIdx.x;
         tally.val = reinterpret_cast<double *>(lst + (size_t)a.tlist * blockDim.x * sizeof(int2)) + threadIdx.x;
         tally.stride = (int)blockDim.x;
@@ -415,10 +453,9 @@ k_event(EvArgs<R> a) {
         bool done = false;
         uint32_t qpos = 0;
         if (have) {
-            Engine<R, StreamAt, Tally, !PHOTON && sizeof(R) == 4> e{constant(a.t), constant(a.g), rng, tally,
-                                                                          {0, 0, 0, 0, 0, 0, 0}, COUNT};
+            Engine<R, StreamAt, Tally, ST> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
             e.nsplit = a.nsplit;          // roulette of the photons that charged particles produce
-            e.eb = eb;
+            e.lds = lds;
             if (PHOTON) {
                 d = a.delta ? e.photon_delta(p, q) : e.photon(p, q);
             } else {
@@ -485,9 +522,11 @@ k_event(EvArgs<R> a) {
 // wave).  Each product gets a random stream of its own, keyed by the
 // photon's stream and its draw position after the interaction; the second
 // product of a pair by the complement of the stream.
-template <class R, bool COUNT>
+template <class R, bool COUNT, int ST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 k_event_split(EvArgs<R> a) {
+    extern __shared__ __align__(16) unsigned char omc_lds[];
+    const Staged<R> lds = stage<R, ST>(a, omc_lds);
     const long long n = (long long)*a.n_in;
     const int ns = a.nsplit;
     const bool takes = (int)(threadIdx.x & 63) < lane_share(n, a.waves);
@@ -514,15 +553,16 @@ k_event_split(EvArgs<R> a) {
             tally.init(a.endep + (size_t)slot * a.slot_stride,
                        a.touched ? a.touched + (size_t)slot * a.touch_stride : nullptr);
         }
-        Engine<R, StreamAt, TallyAtomic> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
+        Engine<R, StreamAt, TallyAtomic, ST> e{constant(a.t), constant(a.g), rng, tally, {0, 0, 0, 0, 0, 0, 0}, COUNT};
         e.nsplit = ns;
+        e.lds = lds;
         // set-up of the split (src/ompmc.c:1900-1940)
         bool live = have, surv = false;
         R eig = (R)0, gle = (R)0, eta = (R)0, d_eta = (R)0, dpmfp_old = (R)0, wtsave = (R)0;
         int i_survive = -1, imed = -1, lgle = 0;
         R cohfac = (R)0, gmfp = (R)0;
         Part<R> save = p;
-        typename Engine<R, StreamAt, TallyAtomic>::SplitXs xs;
+        typename Engine<R, StreamAt, TallyAtomic, ST>::SplitXs xs;
         if (live) {
             if (COUNT) e.cnt.nphoton++;
             imed = e.medium(p);

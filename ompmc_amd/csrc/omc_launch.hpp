@@ -38,7 +38,9 @@ template <class R> struct EvLaunch {
     int nsplit;                  // photon splitting factor; > 1 transports photons with k_event_split
     int graph;                   // 1: untimed chunks of rounds replay a HIP graph
     const CBin<R> *ebin;         // the electron half of the charged bins (Tables::cbin)
-    int eb_words;                // > 0: the charged kernel copies it to LDS (16-byte words)
+    int eb_words;                // its size in 16-byte words where the charged kernel copies it to LDS, else 0
+    int st_charged, st_split;    // tables the charged kernel and the splitting kernel stage in LDS
+    LdsLayout lds_charged, lds_split;
     int tlist;                   // deposit-list entries per charged-kernel lane in LDS (0: direct atomics)
     SrcArgs<R> src;              // source of the job (ctl and out are set per round)
     int grid_event, grid_charged, grid_source;   // workgroups: photon kernels, charged kernel, source

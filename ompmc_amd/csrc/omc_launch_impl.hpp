@@ -69,6 +69,22 @@ template <class R> struct RoundCall {
     }
 };
 
+// The transport kernel of part 1 (photons; split: the splitting kernel) or 2
+// (charged particles) with the tables of st staged in LDS.
+template <class R> const void *event_kernel(int part, bool split, bool count, int st) {
+#define OMC_FN(...) reinterpret_cast<const void *>(&__VA_ARGS__)
+    if (part == 1 && split)
+        return count ? OMC_FN(k_event_split<R, true, 0>)
+                     : st ? OMC_FN(k_event_split<R, false, ST_GEOM>) : OMC_FN(k_event_split<R, false, 0>);
+    if (part == 1) return count ? OMC_FN(k_event<R, true, true, 0>) : OMC_FN(k_event<R, true, false, 0>);
+    if (count) return OMC_FN(k_event<R, false, true, 0>);
+    // FP64 bins are not staged (twice the size, and the kernel has no room to gain from them)
+    if constexpr (std::is_same<R, float>::value)
+        if (st & ST_BINS) return OMC_FN(k_event<R, false, false, ST_GEOM | ST_BINS>);
+    return st ? OMC_FN(k_event<R, false, false, ST_GEOM>) : OMC_FN(k_event<R, false, false, 0>);
+#undef OMC_FN
+}
+
 template <class R> void round_call(const EvLaunch<R> &L, long r, int part, bool count, RoundCall<R> &c) {
     const int par = (int)(r & 1), nx = 1 - par;
     c.part = part;
@@ -104,22 +120,19 @@ template <class R> void round_call(const EvLaunch<R> &L, long r, int part, bool 
         a.delta = L.delta;
         a.nsplit = L.nsplit > 1 ? L.nsplit : 1;
         a.ebin = L.ebin;
-        a.eb_words = part == 2 ? L.eb_words : 0;
-        a.tlist = part == 2 ? L.tlist : 0;
+        // (the counting kernels read every table in device memory)
+        const int st = count ? 0 : part == 2 ? L.st_charged : a.nsplit > 1 ? L.st_split : 0;
+        const bool list = part == 2 && L.tlist > 0;
+        a.eb_words = L.eb_words;
+        a.tlist = list ? L.tlist : 0;
+        a.lds = part == 2 ? L.lds_charged : L.lds_split;
+        if (st == 0) a.lds.list = 0;
         a.waves = part == 2 ? L.waves_charged : L.waves_event;
-        c.shmem = (unsigned)a.eb_words * 16u + (unsigned)a.tlist * c.block.x * 16u;
+        c.shmem = st ? (unsigned)a.lds.bytes : list ? (unsigned)a.tlist * c.block.x * 16u : 0u;
         a.in = L.pool[par][part - 1];
         a.n_in = &L.ctl->cnt[par][part - 1];
         a.claim = &L.ctl->claim[par][part - 1];
-        if (part == 1 && a.nsplit > 1)
-            c.fn = count ? reinterpret_cast<const void *>(&k_event_split<R, true>)
-                         : reinterpret_cast<const void *>(&k_event_split<R, false>);
-        else if (part == 1)
-            c.fn = count ? reinterpret_cast<const void *>(&k_event<R, true, true>)
-                         : reinterpret_cast<const void *>(&k_event<R, true, false>);
-        else
-            c.fn = count ? reinterpret_cast<const void *>(&k_event<R, false, true>)
-                         : reinterpret_cast<const void *>(&k_event<R, false, false>);
+        c.fn = event_kernel<R>(part, a.nsplit > 1, count, st);
         c.grid = dim3(part == 2 ? L.grid_charged : L.grid_event);
     } else {
         c.ctl = L.ctl;
@@ -133,25 +146,7 @@ template <class R> void round_call(const EvLaunch<R> &L, long r, int part, bool 
 template <class R> hipError_t launch_round_part(const EvLaunch<R> &L, long r, int part, bool count, hipStream_t st) {
     RoundCall<R> c;
     round_call(L, r, part, count, c);
-    if (part == 0) {
-        hipLaunchKernelGGL((k_source<R>), c.grid, c.block, 0, st, c.src);
-    } else if (part == 1 || part == 2) {
-        if (c.fn == reinterpret_cast<const void *>(&k_event_split<R, true>))
-            hipLaunchKernelGGL((k_event_split<R, true>), c.grid, c.block, 0, st, c.ev);
-        else if (c.fn == reinterpret_cast<const void *>(&k_event_split<R, false>))
-            hipLaunchKernelGGL((k_event_split<R, false>), c.grid, c.block, 0, st, c.ev);
-        else if (c.fn == reinterpret_cast<const void *>(&k_event<R, true, true>))
-            hipLaunchKernelGGL((k_event<R, true, true>), c.grid, c.block, 0, st, c.ev);
-        else if (c.fn == reinterpret_cast<const void *>(&k_event<R, true, false>))
-            hipLaunchKernelGGL((k_event<R, true, false>), c.grid, c.block, 0, st, c.ev);
-        else if (c.fn == reinterpret_cast<const void *>(&k_event<R, false, true>))
-            hipLaunchKernelGGL((k_event<R, false, true>), c.grid, c.block, c.shmem, st, c.ev);
-        else
-            hipLaunchKernelGGL((k_event<R, false, false>), c.grid, c.block, c.shmem, st, c.ev);
-    } else {
-        hipLaunchKernelGGL(k_round_end, c.grid, c.block, 0, st, c.ctl, c.par);
-    }
-    return hipGetLastError();
+    return hipLaunchKernel(c.fn, c.grid, c.block, c.bind(), c.shmem, st);
 }
 
 // A graph of rounds r0 .. r0+nround-1, built node by node (no stream
