@@ -57,17 +57,16 @@ int device_cus(int dev) {
 }
 
 // ------------------------------------------------------------------ event-form state
-// Condensed-history steps between lane refills.  Whole 1960-beamlet plan,
-// interleaved-bin build, best of three: 8 -> 17.2, 12 -> 18.2, 16 -> 17.7 M
-// histories/s (with 1 M or 2 M in flight, and 16, 24 or 32 turns, all
-// within 1% of each other at 12).  With the two-band charged queue, 16 against
-// 12: 1960-beamlet plan FP32 22.9 against 22.5 M, FP64 12.4 against 12.6 M;
-// 10,044-beamlet plan at 3e8 histories FP32 14.2 against 15.2 M.
-constexpr int DEFAULT_BUDGET = 12;
-// Refills an electron may hold its lane in one round before it is requeued.
-// Measured on the 1960-beamlet plan (1 M in flight): 12 -> 12.0, 16 -> 12.3,
-// 24 -> 12.5, 64 -> 11.2, no limit -> 9.7 M histories/s.
-constexpr int DEFAULT_TURNS = 24;
+// Condensed-history steps between lane refills, and refills an electron may
+// hold its lane in one round before it is requeued (ms; 1e7 histories on the
+// 128^3 slab / 2e5 electrons on a CT / nsplit 20 / 1e6 FP64 histories on 60^3
+// water): 4 x 36 426/67.8/82.2/51.6, 6 x 24 400/66.0/80.2/49.9, 6 x 16
+// 389/68.3/77.3/49.3, 8 x 18 389/66.1/77.7/51.3, 8 x 12 376/68.6/76.6/50.9, 12 x 12
+// 382/66.6/79.9/52.3, 12 x 24 441/65.4/92.5/50.5.  A refill's loads and atomics
+// speak for long stays, the lanes that idle until it and the tracks that
+// hold a launch open for short ones.
+constexpr int DEFAULT_BUDGET = 8;
+constexpr int DEFAULT_TURNS = 18;
 // Workgroups per compute unit of the persistent event kernels.  Whole c3
 // plan, best of three (M histories/s), charged x photon: 8 x 8 21.9,
 // 2 x 8 22.0, 2 x 4 22.2, 4 x 4 21.9 -- within run-to-run noise.

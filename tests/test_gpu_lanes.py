@@ -34,3 +34,19 @@ def test_dose_independent_of_lane_share(slab, form, nsplit, charge, precision):
         assert spread[2].errors == 0 and packed[2].errors == 0
         for a, b in zip(spread[:2], packed[:2]):
             assert np.allclose(a, b, rtol=1e-10, atol=1e-12 * b.max()), nper
+
+
+def test_vacuum_crossing_independent_of_yields():
+    """An electron crosses a vacuum layer voxel by voxel; where the routine
+    yields to the wave's refill does not change its track, also when the
+    medium behind the layer is the one before it (the reference then goes on to
+    an interaction)."""
+    ph_h = P.vacuum_gap_phantom(12, 0.5)
+    c = omc.Context(ph_h.media)
+    ph = c.phantom(ph_h)
+    kw = dict(collimator=(-1, 1, -1, 1), charge=-1, precision=omc.FP64, form=omc.FORM_EVENT, seed=23)
+    ref = c.run_dosxyz(ph, omc.Spectrum.mono(6.0), 500, 2, electron_budget=1000, electron_turns=-1, **kw)[0]
+    for opts in (dict(electron_budget=1), dict(electron_budget=3, electron_turns=1), dict()):
+        a = c.run_dosxyz(ph, omc.Spectrum.mono(6.0), 500, 2, **opts, **kw)[0]
+        assert np.allclose(a, ref, rtol=1e-10, atol=1e-12 * ref.max()), opts
+    c.close()
