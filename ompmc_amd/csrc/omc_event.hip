@@ -104,7 +104,7 @@ constexpr size_t MAX_LDS_PER_GROUP = 80 * 1024;
 // has not drained by then is reported as a step-guard error.
 long max_rounds(long long nhist, long long target) { return 65536L + 8L * (long)(nhist / std::max(target, 1LL)); }
 
-template <class R> size_t pool_entry_bytes() { return sizeof(R) * 10 + sizeof(int) * 6 + 4 + 8 + 16; }
+template <class R> size_t pool_entry_bytes() { return sizeof(uint4) * POOL_VECS<R>; }
 
 template <class R> size_t event_bytes(long long target) {
     return (size_t)4 * (size_t)(8 * target) * pool_entry_bytes<R>() + sizeof(EvCtl);
@@ -146,14 +146,8 @@ template <class R> struct EvState {
             return omc_seterr(OMC_ERR_NOMEM, "event pools for %lld particles exceed 2^31 entries", cap);
         for (int p = 0; p < 2; p++)
             for (int k = 0; k < 2; k++) {
-                Pool<R> &P = pool[p][k];
-                R **fr[10] = {&P.e, &P.x, &P.y, &P.z, &P.u, &P.v, &P.w, &P.wt, &P.demfp, &P.sig0};
-                for (R **f : fr) *f = A.alloc_n<R>(cap);
-                int **fi[6] = {&P.ix, &P.iy, &P.iz, &P.iq, &P.phase, &P.slot};
-                for (int **f : fi) *f = A.alloc_n<int>(cap);
-                P.ctr = A.alloc_n<uint32_t>(cap);
-                P.stream = A.alloc_n<uint64_t>(cap);
-                P.rs = A.alloc_n<uint4>(cap);
+                pool[p][k].base = A.alloc_n<uint4>((size_t)cap * POOL_VECS<R>);
+                pool[p][k].cap = cap;
             }
         ctl = A.alloc_n<EvCtl>(1);
         if (!A.ok) return omc_seterr(OMC_ERR_NOMEM, "event pools for %lld particles do not fit", cap);
