@@ -44,7 +44,8 @@ struct DevArena {
 };
 
 // Block cache of the current device (see DevArena).  devcache_held() is the
-// memory it holds for reuse; devcache_trim() returns all of it to the runtime.
+// memory it holds for reuse; devcache_trim() returns to the runtime all of it
+// that shares no allocation with a block in use.
 void *devcache_alloc(size_t n, size_t *got);
 void devcache_free(void *p, size_t n);
 size_t devcache_held();
