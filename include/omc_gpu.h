@@ -123,8 +123,8 @@ typedef struct omc_run_opts {
     int grid, block;        /* 0 = automatic */
     int count_events;       /* 1: fill the event counters and per-kernel times of omc_run_stats;
                                2: per-kernel times only (events around every transport kernel) */
-    int64_t event_target;   /* event form: particles in flight per round (0 = automatic: 4096 per compute
-                               unit, four times that with nsplit > 1) */
+    int64_t event_target;   /* event form: particles in flight per round (0 = automatic: 16384 per compute
+                               unit, 4096 where several streams or server requests share the device) */
     int electron_budget;    /* event form: condensed-history steps per charged-particle event (0 = automatic) */
     int group;              /* Dij: beamlets transported together (0 = as many as hbm_budget allows,
                                1 = one beamlet at a time, the reference's loop order) */
@@ -133,7 +133,7 @@ typedef struct omc_run_opts {
     int voxel_walk;         /* event form: 1 = photons fly voxel by voxel as the reference's photon()
                                does; 0 = delta tracking with the phantom's majorant (same distribution) */
     int electron_turns;     /* event form: refills of electron_budget steps an electron may hold its lane
-                               within one round before it is requeued (0 = automatic: 18, -1 = no limit) */
+                               within one round before it is requeued (0 = automatic: 30, -1 = no limit) */
     int batches_per_job;    /* event form: batches transported together, each into tallies of its own
                                (0 = as many as the memory budget holds, 1 = one batch per job) */
     int streams;            /* event-form Dij: beamlet groups transported concurrently, each on its own

@@ -60,13 +60,12 @@ int device_cus(int dev) {
 // Condensed-history steps between lane refills, and refills an electron may
 // hold its lane in one round before it is requeued (ms; 1e7 histories on the
 // 128^3 slab / 2e5 electrons on a CT / nsplit 20 / 1e6 FP64 histories on 60^3
-// water): 4 x 36 426/67.8/82.2/51.6, 6 x 24 400/66.0/80.2/49.9, 6 x 16
-// 389/68.3/77.3/49.3, 8 x 18 389/66.1/77.7/51.3, 8 x 12 376/68.6/76.6/50.9, 12 x 12
-// 382/66.6/79.9/52.3, 12 x 24 441/65.4/92.5/50.5.  A refill's loads and atomics
-// speak for long stays, the lanes that idle until it and the tracks that
-// hold a launch open for short ones.
-constexpr int DEFAULT_BUDGET = 8;
-constexpr int DEFAULT_TURNS = 18;
+// water, the first with 4 M in flight): 3 x 48 185/57.6/67.9/35.4, 4 x 36
+// 189/58.0/66.4/36.3, 4 x 24 189/59.2/63.9/37.1, 6 x 16 201/60.5/64.8/38.4, 8 x 18
+// 214/58.9/69.2/38.1, 12 x 12 243/60.4/74.4/43.0.  A short stay refills the lanes
+// whose particles have ended; a refill costs one atomic's and a few loads' wait.
+constexpr int DEFAULT_BUDGET = 4;
+constexpr int DEFAULT_TURNS = 30;
 // Workgroups per compute unit of the persistent event kernels.  Whole c3
 // plan, best of three (M histories/s), charged x photon: 8 x 8 21.9,
 // 2 x 8 22.0, 2 x 4 22.2, 4 x 4 21.9 -- within run-to-run noise.
@@ -110,15 +109,17 @@ template <class R> size_t event_bytes(long long target) {
     return (size_t)4 * (size_t)(8 * target) * pool_entry_bytes<R>() + sizeof(EvCtl);
 }
 
-// Particles in flight: 4096 per compute unit.  On the 1960-beamlet plan the
-// rate is flat from 1 M to 2 M in flight (12.3-12.6 M histories/s) and falls
-// below (10.1 M at 256 k, 12.0 M at 512 k) and above (11.6 M at 4 M).
-// With photon splitting a history carries nsplit times more electrons, and
-// rounds are fewer and fuller with four times the particles in flight: at
-// nsplit 20 on every 20th beamlet 1.40 s at 1 M, 1.13 s at 2 M, 1.05 s at
-// 4 M and 1.04 s at 8 M (15.3 s against 16.3 s on the whole plan).
-long long default_target(int dev, int nsplit = 1) {
-    return (long long)device_cus(dev) * 4096 * (nsplit > 1 ? 4 : 1);
+// Particles in flight.  Every launch ends with the electrons that started last
+// while the device empties, so fewer and fuller rounds pay where one stream
+// has the device to itself: 16384 per compute unit (1e7 histories on the 128^3
+// slab at 1 M, 2 M and 4 M in flight: 246, 208 and 189 ms; a 196-beamlet FP64
+// matrix 118, 108, 109).  Where several streams overlap one another's ends,
+// 4096 (the 1960-beamlet plan on three streams at 0.5, 1, 2 and 4 M: 510, 478, 492
+// and 523 ms, the larger pools leaving less memory for tallies).  With photon
+// splitting a history carries nsplit times more electrons: 16384 in any case
+// (nsplit 20 on every 20th beamlet at 1, 2, 4 and 8 M: 1.40, 1.13, 1.05, 1.04 s).
+long long default_target(int dev, int nsplit, bool alone) {
+    return (long long)device_cus(dev) * 4096 * (nsplit > 1 || alone ? 4 : 1);
 }
 
 // run_job's code for a pool overflow: the caller zeroes the job's tallies,
@@ -475,9 +476,14 @@ int omc_run_dosxyz_event(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const o
     // order afterwards, so the result is the batch-by-batch one while the
     // job drains its longest tracks once instead of once per batch.
     const int nbj = batches_per_job(o, nbatch, (size_t)nreg * sizeof(double));
-    long long tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit);
+    long long tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit, true);
     if (tgt > 4 * (long long)nper * nbj) tgt = std::max<long long>(4 * (long long)nper * nbj, 64);
     int rc = S.alloc(tgt);
+    if (rc && o->event_target <= 0 && tgt > default_target(c->device, o->nsplit, false)) {
+        S.A.release();               // little memory left: the smaller pools
+        S.A.ok = true;
+        rc = S.alloc(default_target(c->device, o->nsplit, false));
+    }
     if (rc) return rc;
     double *d_e = A.alloc_n<double>((size_t)nbj * nreg), *d_s = A.alloc_n<double>(nreg),
            *d_s2 = A.alloc_n<double>(nreg);
@@ -1040,7 +1046,7 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
     D.nper = beamlet_nper(bix, nbatch);
     for (long n : D.nper)
         if (n >= (1L << 32)) return omc_seterr(OMC_ERR_LIMIT, "more than 2^32 histories per batch of a beamlet");
-    D.tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit);
+    D.tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit, false);
     // lanes: up to three for an event-form run of several groups (o->streams
     // pins the number), each planned on its share of the memory budget.  On
     // the 1960-beamlet plan at 96 GiB: 1 lane 7.2, 2 lanes 10.1, 3 lanes
@@ -1051,6 +1057,12 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
     int NL = 1;
     if (D.event) NL = o->streams > 0 ? o->streams : std::min(3, (nbix + plan.G - 1) / plan.G);
     if (NL > 1) dij_plan(o, nreg, nbix, nbatch, D.tgt, budget / NL, plan);
+    if (NL == 1 && D.event && o->event_target <= 0) {
+        // one stream: the larger pools where they leave the plan as it is
+        const long long big = default_target(c->device, o->nsplit, true);
+        DijPlan p;
+        if (dij_plan(o, nreg, nbix, nbatch, big, budget, p) <= budget && p.G == plan.G && p.nbj == plan.nbj) D.tgt = big;
+    }
     D.G = plan.G;
     D.NBJ = plan.nbj;
     // every batch of a group in one job: the batch statistics fold into the
@@ -1402,7 +1414,7 @@ size_t request_bytes(omc_server *s, const omc_request &r) {
     const omc_phantom_desc &p = r.phantom;
     long nreg = (long)p.nx * p.ny * p.nz + 1;
     size_t b = omc_phantom_bytes(&p);
-    long long tgt = default_target(s->ctx->device, r.nsplit);
+    long long tgt = default_target(s->ctx->device, r.nsplit, false);
     size_t ev = r.precision == OMC_FP64 ? event_bytes<double>(tgt) : event_bytes<float>(tgt);
     // dose: every batch in one job, each with its own tallies
     if (r.kind == OMC_REQ_DOSE) return b + (size_t)(r.nbatch + 2) * nreg * 8 + ev;
@@ -1434,6 +1446,9 @@ void run_request(omc_server *s, omc_server::Req *q) {
     o.form = OMC_FORM_EVENT;
     o.seed = q->r.seed;
     o.nsplit = q->r.nsplit;
+    // concurrent requests overlap one another's round ends; the admission
+    // counts these pools
+    if (q->r.kind == OMC_REQ_DOSE) o.event_target = default_target(c->device, o.nsplit, false);
     o.batches_per_job = q->r.kind == OMC_REQ_DOSE ? q->r.nbatch : 0;
     // concurrent requests already overlap one another's drains; extra group
     // streams per Dij request only contend for the hardware queues (served
