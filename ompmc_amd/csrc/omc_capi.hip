@@ -402,7 +402,10 @@ template <class R> static int upload_tables(omc_ctx *c, DevArena &A, Tables<R> &
     T.cbin = A.upload(cb);
     T.cb_stride = stride;
     std::vector<MsBin<R>> msb(OMC_NMS);
-    for (size_t n = 0; n < (size_t)OMC_NMS; n++) msb[n] = MsBin<R>{(R)h.wms[n], h.ims[n], (R)h.fms[n], (R)h.ums[n]};
+    for (size_t n = 0; n < (size_t)OMC_NMS; n++) {
+        const size_t row = n / (MXU_MS + 1) * (MXU_MS + 1);
+        msb[n] = MsBin<R>{(R)h.wms[n], (R)h.ums[n], (R)h.ums[row + std::min(std::max(h.ims[n], 0), MXU_MS)]};
+    }
     T.ms = A.upload(msb);
     T.b2spin_min = (R)h.b2spin_min; T.dbeta2i = (R)h.dbeta2i; T.espml = (R)h.espml; T.dleneri = (R)h.dleneri;
     T.dqq1i = (R)h.dqq1i; T.dllambi = (R)h.dllambi; T.dqmsi = (R)h.dqmsi;
