@@ -716,7 +716,7 @@ static int run_dosxyz_history(omc_ctx *c, hipStream_t stream, PhantomDev *pd, co
     float ms = 0.f;
     const int hblock = o->block > 0 ? o->block : 256;
     // the largest launch of the run (the particle stacks of nsplit > 8 cover it)
-    int max_grid = o->grid > 0 ? o->grid : (int)std::min<int64_t>((nper + hblock - 1) / hblock, 2048);
+    int max_grid = hist_grid(c->device, nper, o, a.waves);
     int err[4] = {0, 0, 0, 0};
     auto wall0 = std::chrono::steady_clock::now();
     if (!A.ok) { rc = omc_seterr(OMC_ERR_NOMEM, "device allocation failed"); goto done; }
@@ -760,10 +760,7 @@ static int run_dosxyz_history(omc_ctx *c, hipStream_t stream, PhantomDev *pd, co
         a.hist_base = (long)b * nper;
         a.replay_off = d_off ? d_off + (long)b * nper : nullptr;
         HIPCHK(hipMemsetAsync(d_next, 0, sizeof(unsigned long long), stream));
-        int block = hblock;
-        long want = (nper + block - 1) / block;
-        int grid = o->grid > 0 ? o->grid : (int)(want < 2048 ? want : 2048);
-        if (grid > max_grid) grid = max_grid;
+        const int block = hblock, grid = max_grid;
         if (o->count_events) HIPCHK(hipEventRecord(kev[2 * b], stream));
         HIPCHK(launch_history<R>(a, o->rng == OMC_RNG_REPLAY ? RNG_REPLAY : RNG_STREAMS, (o->count_events & 1) != 0,
                                  grid, block, stream));

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
@@ -170,6 +171,23 @@ template <class R> inline int make_dosxyz_src(DevArena &A, const PhantomDev *pd,
 // it counts as stuck; max_particle_steps sets it, 0 means 10^8.
 inline long hist_max_steps(const omc_run_opts *o) {
     return o->max_particle_steps > 0 ? (long)o->max_particle_steps : 100000000L;
+}
+
+// Workgroups of a history-form launch of n histories with the automatic shape:
+// enough lanes for all, and where the device holds more wavefronts (two a
+// SIMD, by the kernel's registers) than they fill, a wavefront for every
+// history up to that many (waves, see lane_share).  Launches of a given shape
+// and the splitting kernel keep 64 lanes a wavefront.
+inline int hist_grid(int device, int64_t n, const omc_run_opts *o, int &waves) {
+    const int block = o->block > 0 ? o->block : 256;
+    const int64_t full = std::min<int64_t>((n + block - 1) / block, 2048);
+    waves = 0;
+    if (o->grid > 0) return o->grid;
+    if (o->block > 0 || o->nsplit > 1) return (int)full;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) cus = 256;
+    waves = cus * 8;
+    return (int)std::max<int64_t>(full, (std::min<int64_t>(n, waves) + 3) / 4);
 }
 
 // Device-memory particle stacks for history-form splitting beyond the

@@ -812,7 +812,7 @@ template <class R> int dij_lane_init(DijRun<R> &D, DijLane<R> &l) {
             for (int b = g0; b < std::min(D.nbix, g0 + G); b++) t += D.nper[b];
             maxlaunch = std::max(maxlaunch, t);
         }
-        l.max_grid = o->grid > 0 ? o->grid : (int)std::min<long long>((maxlaunch + hblock - 1) / hblock, 2048);
+        l.max_grid = std::max(hist_grid(D.c->device, maxlaunch, o, H.waves), 1);
         int rc = alloc_split_stacks<R>(A, H, o->nsplit, hblock, l.max_grid);
         if (rc) return rc;
     }
@@ -915,9 +915,8 @@ template <class R> int dij_lane_group(DijRun<R> &D, DijLane<R> &l, int gi) {
                     CK(hipStreamSynchronize(stream));   // rs/re go out of scope
                 }
                 CK(hipMemsetAsync(D.d_next, 0, sizeof(unsigned long long), stream));
-                int block = o->block > 0 ? o->block : 256;
-                long want = (njob + block - 1) / block;
-                int grid = o->grid > 0 ? o->grid : (int)std::min<long>(want, 2048);
+                const int block = o->block > 0 ? o->block : 256;
+                int grid = hist_grid(D.c->device, njob, o, H.waves);
                 if (grid > l.max_grid) grid = l.max_grid;
                 if (D.timing) CK(hipEventRecord(ev.ev[0], stream));
                 CK(launch_history<R>(H, D.replay ? RNG_REPLAY : RNG_STREAMS, D.count, grid, block, stream));

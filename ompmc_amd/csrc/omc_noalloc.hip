@@ -131,8 +131,7 @@ int run_noalloc(omc_ctx *c, PhantomDev *pd, const omc_dosxyz_source_desc *src, i
         a.hist_base = (long)b * nper;
         HIPCHK(zero64(d_next, sizeof(unsigned long long), stream));
         const int block = o->block > 0 ? o->block : 256;
-        const long want = (nper + block - 1) / block;
-        const int grid = o->grid > 0 ? o->grid : (int)(want < 2048 ? want : 2048);
+        const int grid = hist_grid(c->device, nper, o, a.waves);
         HIPCHK(launch_history<R>(a, RNG_STREAMS, (o->count_events & 1) != 0, grid, block, stream));
         HIPCHK(launch_accumulate(d_e, d_sum, d_sum2, nreg, 1.0, d_ebal + EB_DEPOSIT, stream));
     }

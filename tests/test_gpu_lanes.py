@@ -22,7 +22,7 @@ def slab():
     c.close()
 
 
-@pytest.mark.parametrize("form", [omc.FORM_EVENT], ids=["event"])
+@pytest.mark.parametrize("form", [omc.FORM_EVENT, omc.FORM_HISTORY], ids=["event", "history"])
 @pytest.mark.parametrize("nsplit,charge", [(1, 0), (4, 0), (1, -1)], ids=["photons", "split", "electrons"])
 @pytest.mark.parametrize("precision", [omc.FP32, omc.FP64], ids=["fp32", "fp64"])
 def test_dose_independent_of_lane_share(slab, form, nsplit, charge, precision):
