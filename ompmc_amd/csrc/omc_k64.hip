@@ -68,13 +68,19 @@ __device__ __forceinline__ void dij_finish_voxel(double acc, double acc2, double
 // are zero, and the reference adds 0 and 0^2.  Dose and variance are written
 // only in tiles some batch touched (`any` marks them for the selection); in
 // the others the dose is zero, and so is the variance carried on.  Also
-// per-block maxima, the energy deposited (raw tallies, the EB_DEPOSIT term)
-// and the beamlet-summed dose and plan variance.
+// per-block maxima (zeroed before the launch), the energy deposited (raw
+// tallies, the EB_DEPOSIT term) and the beamlet-summed dose and plan variance.
+//
+// Nearly all of a tile's (batch, beamlet) marks are unset, and reading them is
+// what the kernel waits for: a wave reads 64 of them at once, for several
+// beamlets, and the next 64 while it folds, where it read them one after
+// another; and its waves no longer meet twice a beamlet for the block's
+// maximum.  1960-beamlet plan 543 -> 505 ms, 50 beamlets on 13 M voxels 60.8 ->
+// 56.3 ms, 196 FP64 beamlets 123 -> 121 ms.
 __global__ void __launch_bounds__(DIJ_BLOCK)
 k_dij_fold_finish(double *e, uint8_t *touched, int ng, int nbatch, long nreg, long ntile, const double *nper,
                   double *dose, double *var, uint8_t *any, double *carry, const double *mass, const double *rho,
                   double *blockmax, double *tot_dose, double *tot_var, double *dep) {
-    __shared__ double lds[DIJ_BLOCK / 64];
     const int lane = threadIdx.x & 63;
     const long t = (long)blockIdx.x * (DIJ_BLOCK / 64) + (threadIdx.x >> 6);
     const bool tile_in = t < ntile;
@@ -83,44 +89,100 @@ k_dij_fold_finish(double *e, uint8_t *touched, int ng, int nbatch, long nreg, lo
     const double m = in ? mass[irl - 1] : 1.0, r = in ? rho[irl - 1] : 1.0;
     const double factor = 1.602E-10 / (m);
     double c = in ? carry[irl] : 0.0, td = 0.0, tv = 0.0, raw = 0.0;
-    for (int s = 0; s < ng; s++) {
-        const double np = nper[s];
-        double acc = 0.0, acc2 = c, acc2raw = 0.0;
-        bool hit = false;
-        for (int k = 0; k < nbatch; k++) {
-            const long slot = (long)k * ng + s;
-            uint8_t *mark = touched + slot * ntile + t;
-            if (tile_in && *mark) {                    // the same for every lane of the wave
-                hit = true;
-                double x = 0.0;
+    // lane l holds the mark of batch l % nbatch of beamlet s0 + l / nbatch (of
+    // batch k0 + l of beamlet s0 where a beamlet has more batches than lanes)
+    const int per = nbatch <= 64 ? 64 / nbatch : 1;
+    const int ds = nbatch <= 64 ? lane / nbatch : 0, dk = lane - ds * nbatch * (nbatch <= 64);
+    const unsigned long long batches = nbatch >= 64 ? ~0ull : (1ull << nbatch) - 1ull;
+    auto mark_at = [&](int s0, int k0) -> uint8_t * {
+        if (!tile_in || ds >= per || s0 + ds >= ng || k0 + dk >= nbatch) return nullptr;
+        return touched + ((long)(k0 + dk) * ng + s0 + ds) * ntile + t;
+    };
+    // folds the marked batches of `mask` (bit j: batch k0 + j) of beamlet s, in
+    // batch order, four slots' loads in flight together
+    double acc = 0.0, acc2 = 0.0, acc2raw = 0.0, np = 1.0;
+    auto fold = [&](int s, int k0, unsigned long long mask) {
+        while (mask) {
+            double x[4];
+            double *pe[4];
+            int n = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                x[j] = 0.0;
+                pe[j] = nullptr;
+                if (!mask) continue;
+                const int k = k0 + __ffsll(mask) - 1;
+                mask &= mask - 1;
+                n++;
                 if (irl < nreg) {
-                    double *pe = e + slot * nreg + irl;
-                    x = *pe;
-                    if (x != 0.0) *pe = 0.0;
+                    pe[j] = e + ((long)k * ng + s) * nreg + irl;
+                    x[j] = *pe[j];
                 }
-                raw += x;
-                x /= np;
-                acc += x;
-                acc2 += x * x;
-                acc2raw += x * x;
-                if (lane == 0) *mark = 0;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j >= n) continue;
+                if (x[j] != 0.0) *pe[j] = 0.0;
+                raw += x[j];
+                const double v = x[j] / np;
+                acc += v;
+                acc2 += v * v;
+                acc2raw += v * v;
             }
         }
-        double dd = 0.0;
-        if (in) {
-            double vv, u0;
-            dij_finish_voxel(acc, acc2, acc2raw, factor, r, nbatch, dd, vv, u0);
-            c = vv;
-            td += dd;
-            tv += u0;
+    };
+    uint8_t *mark = mark_at(0, 0);
+    bool set = mark && *mark;
+    for (int s0 = 0; s0 < ng; s0 += per) {
+        const unsigned long long marked = __ballot(set);
+        if (set) *mark = 0;
+        // the next beamlets' marks while these are folded
+        mark = s0 + per < ng ? mark_at(s0 + per, 0) : nullptr;
+        set = mark && *mark;
+        const int ns = ng - s0 < per ? ng - s0 : per;
+        if (nbatch <= 64 && !marked) {              // no energy in this tile: dose and variance are zero
+            c = 0.0;
+            if (tile_in && lane < ns) any[(long)(s0 + lane) * ntile + t] = 0;
+            continue;
+        }
+        for (int d = 0; d < ns; d++) {
+            const int s = s0 + d;
+            unsigned long long mask = (marked >> (d * nbatch * (nbatch <= 64))) & batches;
+            bool hit = mask != 0;
+            np = nper[s];
+            acc = acc2raw = 0.0;
+            acc2 = c;
+            fold(s, 0, mask);
+            for (int k0 = 64; k0 < nbatch; k0 += 64) {
+                uint8_t *mk = mark_at(s, k0);
+                const bool st = mk && *mk;
+                if (st) *mk = 0;
+                mask = __ballot(st);
+                hit = hit || mask != 0;
+                fold(s, k0, mask);
+            }
+            double dd = 0.0;
+            if (in) {
+                double vv, u0;
+                dij_finish_voxel(acc, acc2, acc2raw, factor, r, nbatch, dd, vv, u0);
+                c = vv;
+                td += dd;
+                tv += u0;
+                if (hit) {
+                    dose[(long)s * nreg + irl] = dd;
+                    var[(long)s * nreg + irl] = vv;
+                }
+            }
+            if (tile_in && lane == 0) any[(long)s * ntile + t] = hit ? 1 : 0;
             if (hit) {
-                dose[(long)s * nreg + irl] = dd;
-                var[(long)s * nreg + irl] = vv;
+                double bm = dd;
+                for (int off = 32; off > 0; off >>= 1) bm = fmax(bm, __shfl_xor(bm, off));
+                // positive doubles order like their bits
+                if (lane == 0 && bm > 0.0)
+                    atomicMax((unsigned long long *)(blockmax + (long)s * gridDim.x + blockIdx.x),
+                              (unsigned long long)__double_as_longlong(bm));
             }
         }
-        if (tile_in && lane == 0) any[(long)s * ntile + t] = hit ? 1 : 0;
-        const double bm = block_max(dd, lds);
-        if (threadIdx.x == 0) blockmax[(long)s * gridDim.x + blockIdx.x] = bm;
     }
     if (in) {
         carry[irl] = c;
@@ -266,6 +328,8 @@ hipError_t launch_dij_fold_finish(double *e, uint8_t *touched, int ng, int nbatc
                                   const double *rho, double *blockmax, double *tot_dose, double *tot_var, double *dep,
                                   hipStream_t st) {
     const long ntile = dij_ntile(nreg);
+    hipError_t err = hipMemsetAsync(blockmax, 0, sizeof(double) * (size_t)ng * dij_nblk(nreg), st);
+    if (err != hipSuccess) return err;
     hipLaunchKernelGGL(k_dij_fold_finish, dim3(dij_nblk(nreg)), dim3(DIJ_BLOCK), 0, st, e, touched, ng, nbatch, nreg,
                        ntile, nper, dose, var, any, carry, mass, rho, blockmax, tot_dose, tot_var, dep);
     return hipGetLastError();
