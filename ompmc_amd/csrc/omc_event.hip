@@ -521,8 +521,7 @@ int omc_run_dosxyz_event(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const o
         rc = run_job_grow(stream, S, L, (long long)nper * nb, dest, (o->count_events & 1) != 0,
                           o->count_events != 0, js, d_e, (size_t)nb * nreg, d_ebal);
         if (rc) return rc;
-        for (int k = 0; k < nb; k++)
-            CK(launch_accumulate(d_e + (size_t)k * nreg, d_s, d_s2, nreg, 1.0, d_ebal + EB_DEPOSIT, stream));
+        CK(launch_accumulate_job(d_e, nreg, nb, d_s, d_s2, nreg, b0 + nb < nbatch, d_ebal + EB_DEPOSIT, stream));
     }
     CK(hipEventRecord(ev.ev[1], stream));
     CK(hipStreamSynchronize(stream));
