@@ -13,6 +13,7 @@
 #include <mutex>
 #include <vector>
 
+#include "omc_blocks.hpp"
 #include "omc_capi_internal.hpp"
 
 using namespace omc;
@@ -33,129 +34,25 @@ int omc_seterr(int code, const char *fmt, ...) {
 // ------------------------------------------------------------------ device memory
 namespace {
 
-// Device memory of runs, kept for reuse.  A slab is one allocation of the
-// runtime, cut into blocks on demand; a released block joins its free
-// neighbours.  A request takes the smallest free block that holds it and gives
-// back the rest, so runs of different sizes share the same memory.  (Blocks
-// reused whole, by size, piled up: once plans of other sizes had filled the
-// cache, every pass of the next plan mapped and unmapped its tallies anew.  In a
-// process that had run other plans before, a 196-beamlet FP64 plan took 1130 ms
-// a pass against 208 ms alone, 50 beamlets on 13 M voxels 1480 against 95 ms.)
-// Sizes are rounded to 2 MiB.  At most CACHE_MAX bytes stay free: beyond that,
-// slabs without a block in use go back to the runtime, the one unused for
-// longest first.
-struct Slab;
-struct Block {
-    Slab *slab;
-    size_t size;
-    bool free;
+// hipMalloc's memory of the current device
+struct HipMem {
+    int device() {
+        int d = 0;
+        (void)hipGetDevice(&d);
+        return d;
+    }
+    void *get(size_t n) {
+        void *p = nullptr;
+        if (hipMalloc(&p, n) == hipSuccess) return p;
+        (void)hipGetLastError();          // recovered by the caller: keep it from surfacing at the next launch check
+        return nullptr;
+    }
+    void put(void *p) { (void)hipFree(p); }
 };
-struct Slab {
-    char *base;
-    size_t size;
-    size_t used = 0;                 // bytes handed out
-    unsigned long long stamp = 0;    // when it was last drawn on or emptied
-};
-struct DevCache {
-    std::mutex mu;
-    std::map<char *, Block> blocks;                    // every block by address
-    std::multimap<size_t, char *> free;                // the free ones by size
-    std::map<char *, std::unique_ptr<Slab>> slabs;     // by address
-    size_t held = 0;                                   // free bytes
-    unsigned long long clock = 0;
-    void drop_free(std::map<char *, Block>::iterator it) {
-        for (auto f = free.lower_bound(it->second.size); f != free.end() && f->first == it->second.size; ++f)
-            if (f->second == it->first) {
-                free.erase(f);
-                return;
-            }
-    }
-    void add_free(std::map<char *, Block>::iterator it) { free.emplace(it->second.size, it->first); }
-    // the smallest free block of at least n bytes, cut to n.  A small block is
-    // not cut from a much larger one, which another run may need whole while
-    // it is in use.
-    void *take(size_t n) {
-        auto f = free.lower_bound(n);
-        if (f == free.end() || f->first > std::max(64 * n, (size_t)1 << 30)) return nullptr;
-        auto it = blocks.find(f->second);
-        free.erase(f);
-        Block &b = it->second;
-        if (b.size > n) {
-            auto rest = blocks.emplace(it->first + n, Block{b.slab, b.size - n, true}).first;
-            add_free(rest);
-            b.size = n;
-        }
-        b.free = false;
-        b.slab->used += n;
-        b.slab->stamp = ++clock;
-        held -= n;
-        return it->first;
-    }
-    // a slab that is handed out whole
-    void *take_at(void *p) {
-        auto it = blocks.find((char *)p);
-        drop_free(it);
-        it->second.free = false;
-        it->second.slab->used = it->second.size;
-        it->second.slab->stamp = ++clock;
-        held -= it->second.size;
-        return p;
-    }
-    void add_slab(void *p, size_t n) {
-        Slab *s = new Slab{(char *)p, n};
-        slabs[s->base].reset(s);
-        add_free(blocks.emplace(s->base, Block{s, n, true}).first);
-        held += n;
-    }
-    void give(void *p) {
-        auto it = blocks.find((char *)p);
-        if (it == blocks.end() || it->second.free) return;
-        Slab *s = it->second.slab;
-        it->second.free = true;
-        s->used -= it->second.size;
-        s->stamp = ++clock;
-        held += it->second.size;
-        auto next = std::next(it);
-        if (next != blocks.end() && next->second.slab == s && next->second.free) {
-            drop_free(next);
-            it->second.size += next->second.size;
-            blocks.erase(next);
-        }
-        if (it != blocks.begin()) {
-            auto prev = std::prev(it);
-            if (prev->second.slab == s && prev->second.free) {
-                drop_free(prev);
-                prev->second.size += it->second.size;
-                blocks.erase(it);
-                it = prev;
-            }
-        }
-        add_free(it);
-    }
-    // takes the unused slab that has been so for longest out of the cache (null: none)
-    void *evict() {
-        Slab *old = nullptr;
-        for (auto &kv : slabs)
-            if (kv.second->used == 0 && (!old || kv.second->stamp < old->stamp)) old = kv.second.get();
-        if (!old) return nullptr;
-        char *base = old->base;
-        auto it = blocks.find(base);      // an unused slab is one free block
-        drop_free(it);
-        held -= it->second.size;
-        blocks.erase(it);
-        slabs.erase(base);
-        return base;
-    }
-};
-constexpr size_t CACHE_GRAIN = (size_t)2 << 20;
-constexpr size_t CACHE_MAX = (size_t)128 << 30;
-constexpr int CACHE_DEVICES = 64;
 
-DevCache &cache_here() {
-    static DevCache caches[CACHE_DEVICES];
-    int d = 0;
-    (void)hipGetDevice(&d);
-    return caches[(unsigned)d % CACHE_DEVICES];
+DevBlocks<HipMem> &dev_blocks() {
+    static DevBlocks<HipMem> b;
+    return b;
 }
 
 std::mutex pinned_mu;
@@ -163,58 +60,10 @@ std::vector<void *> pinned_free;
 
 }  // namespace
 
-void *devcache_alloc(size_t n, size_t *got) {
-    n = (n + CACHE_GRAIN - 1) / CACHE_GRAIN * CACHE_GRAIN;
-    *got = n;
-    DevCache &C = cache_here();
-    {
-        std::lock_guard<std::mutex> lk(C.mu);
-        if (void *p = C.take(n)) return p;
-    }
-    void *p = nullptr;
-    if (hipMalloc(&p, n) != hipSuccess) {
-        (void)hipGetLastError();          // recovered below: keep it from surfacing at the next launch check
-        devcache_trim();
-        if (hipMalloc(&p, n) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-    }
-    std::lock_guard<std::mutex> lk(C.mu);
-    C.add_slab(p, n);
-    return C.take_at(p);
-}
-
-void devcache_free(void *p, size_t) {
-    DevCache &C = cache_here();
-    std::vector<void *> out;
-    {
-        std::lock_guard<std::mutex> lk(C.mu);
-        C.give(p);
-        while (C.held > CACHE_MAX) {
-            void *s = C.evict();
-            if (!s) break;                // what is left is in slabs that are in use
-            out.push_back(s);
-        }
-    }
-    for (void *s : out) (void)hipFree(s);
-}
-
-size_t devcache_held() {
-    DevCache &C = cache_here();
-    std::lock_guard<std::mutex> lk(C.mu);
-    return C.held;
-}
-
-void devcache_trim() {
-    DevCache &C = cache_here();
-    std::vector<void *> out;
-    {
-        std::lock_guard<std::mutex> lk(C.mu);
-        while (void *s = C.evict()) out.push_back(s);
-    }
-    for (void *s : out) (void)hipFree(s);
-}
+void *devcache_alloc(size_t n, size_t *got) { return dev_blocks().alloc(n, got); }
+void devcache_free(void *p, size_t) { dev_blocks().release(p); }
+size_t devcache_held() { return dev_blocks().held(); }
+void devcache_trim() { dev_blocks().trim(); }
 
 void *pinned_small_alloc() {
     {
