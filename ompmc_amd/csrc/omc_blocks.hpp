@@ -168,10 +168,22 @@ template <class Mem> struct DevBlocks {
         for (void *s : out) mem.put(s);
     }
 
-    size_t held() {
+    // memory that a plan may count on beside what the runtime has free: the
+    // slabs without a block in use, which can go back to it, and the largest
+    // free block of the others (their smaller pieces serve no large request).
+    // A request of at most half of both together is served.
+    size_t reusable() {
         DevCache &C = here();
         std::lock_guard<std::mutex> lk(C.mu);
-        return C.held;
+        size_t idle = 0, piece = 0;
+        for (auto &kv : C.slabs)
+            if (kv.second->used == 0) idle += kv.second->size;
+        for (auto f = C.free.rbegin(); f != C.free.rend(); ++f)
+            if (C.blocks.find(f->second)->second.slab->used != 0) {
+                piece = f->first;
+                break;
+            }
+        return idle + piece;
     }
 
     void trim() {

@@ -62,7 +62,7 @@ std::vector<void *> pinned_free;
 
 void *devcache_alloc(size_t n, size_t *got) { return dev_blocks().alloc(n, got); }
 void devcache_free(void *p, size_t) { dev_blocks().release(p); }
-size_t devcache_held() { return dev_blocks().held(); }
+size_t devcache_reusable() { return dev_blocks().reusable(); }
 void devcache_trim() { dev_blocks().trim(); }
 
 void *pinned_small_alloc() {

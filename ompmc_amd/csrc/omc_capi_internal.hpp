@@ -44,12 +44,13 @@ struct DevArena {
     void release();
 };
 
-// Block cache of the current device (see DevArena).  devcache_held() is the
-// memory it holds for reuse; devcache_trim() returns to the runtime all of it
-// that shares no allocation with a block in use.
+// Block cache of the current device (see DevArena).  devcache_reusable() is the
+// memory a plan may count on beside what the runtime has free; devcache_trim()
+// returns to the runtime all of it that shares no allocation with a block in
+// use.
 void *devcache_alloc(size_t n, size_t *got);
 void devcache_free(void *p, size_t n);
-size_t devcache_held();
+size_t devcache_reusable();
 void devcache_trim();
 // Small pinned host buffers (control-block snapshots), kept for reuse: hipHostFree
 // also synchronises the device.

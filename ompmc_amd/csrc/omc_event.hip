@@ -318,11 +318,11 @@ int run_job(hipStream_t st, EvState<R> &S, EvLaunch<R> &L, long long nhist, int 
     return OMC_OK;
 }
 
-// Half of the device memory that is free or held for reuse by the block cache.
+// Half of the device memory that is free or that the block cache can hand out.
 size_t default_budget() {
     size_t freeb = 0, totalb = 0;
     if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) freeb = (size_t)8 << 30;
-    return (freeb + devcache_held()) / 2;
+    return (freeb + devcache_reusable()) / 2;
 }
 
 // Batches of a dose run transported in one job: o->batches_per_job, else as
@@ -1531,7 +1531,7 @@ extern "C" int omc_server_create(omc_ctx *ctx, int64_t hbm_budget_bytes, int max
         size_t freeb = 0, totalb = 0;
         (void)hipSetDevice(ctx->device);
         if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) freeb = (size_t)8 << 30;
-        freeb += devcache_held();
+        freeb += devcache_reusable();
         hbm_budget_bytes = (int64_t)std::min(freeb * 3 / 4, (size_t)96 << 30);
     }
     s->budget = hbm_budget_bytes;

@@ -121,6 +121,43 @@ static void full_card() {
     EXPECT(B.alloc(90 * GiB, &got) != nullptr);      // every idle byte can go back to the runtime
 }
 
+// half of what a plan counts as free or reusable can be had in one block
+static void reusable() {
+    Cache B;
+    size_t got;
+    std::vector<void *> v;
+    void *whole = B.alloc(80 * GiB, &got);
+    B.release(whole);
+    for (int k = 0; k < 40; k++) v.push_back(B.alloc(2 * GiB, &got));
+    EXPECT(B.mem.live.size() == 1);           // all cut from the one slab
+    for (int k = 0; k < 40; k++)
+        if (k % 4) B.release(v[k]);           // 60 GiB free, in pieces of 6
+    size_t counted = B.mem.total - B.mem.used[0] + B.reusable();
+    EXPECT(B.alloc(counted / 2, &got) != nullptr);
+
+    std::mt19937 g(11);
+    for (int k = 0; k < 300; k++) {
+        Cache C;
+        std::vector<void *> live;
+        for (int j = 0; j < 60; j++) {
+            if (live.size() < 12 && g() % 2) {
+                size_t n = (size_t)1 << (24 + g() % 11);
+                void *p = C.alloc(n + g() % n, &got);
+                if (p) live.push_back(p);
+            } else if (!live.empty()) {
+                size_t i = g() % live.size();
+                C.release(live[i]);
+                live.erase(live.begin() + (long)i);
+            }
+        }
+        const size_t grain = 2 * MiB;
+        counted = C.mem.total - C.mem.used[0] + C.reusable();
+        if (counted / 2 < grain) continue;
+        EXPECT(C.alloc(counted / 2 / grain * grain, &got) != nullptr);
+        consistent(C, 0);
+    }
+}
+
 // any order of requests and releases leaves the lists in agreement
 static void any_order() {
     Cache B;
@@ -148,6 +185,7 @@ int main(int argc, char **argv) {
     const struct { const char *name; void (*fn)(); } checks[] = {
         {"cut_join_evict", cut_join_evict},
         {"full_card", full_card},
+        {"reusable", reusable},
         {"any_order", any_order},
     };
     for (auto &c : checks)
