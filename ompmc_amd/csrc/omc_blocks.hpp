@@ -83,9 +83,10 @@ struct DevCache {
         add_free(blocks.emplace(s->base, Block{s, n, true}).first);
         held += n;
     }
-    void give(void *p) {
+    // false: not a block of this cache that is in use
+    bool give(void *p) {
         auto it = blocks.find((char *)p);
-        if (it == blocks.end() || it->second.free) return;
+        if (it == blocks.end() || it->second.free) return false;
         Slab *s = it->second.slab;
         it->second.free = true;
         s->used -= it->second.size;
@@ -107,6 +108,7 @@ struct DevCache {
             }
         }
         add_free(it);
+        return true;
     }
     // takes the unused slab that has been so for longest out of the cache (null: none)
     void *evict() {
@@ -153,19 +155,25 @@ template <class Mem> struct DevBlocks {
         return C.take_at(p);
     }
 
+    // a block goes back to the cache it is of: the current device's, or
+    // another's where the caller's thread has turned to another device since
     void release(void *p) {
-        DevCache &C = here();
-        std::vector<void *> out;
-        {
-            std::lock_guard<std::mutex> lk(C.mu);
-            C.give(p);
-            while (C.held > CACHE_MAX) {
-                void *s = C.evict();
-                if (!s) break;                // what is left is in slabs that are in use
-                out.push_back(s);
+        const unsigned at = (unsigned)mem.device() % CACHE_DEVICES;
+        for (unsigned k = 0; k < CACHE_DEVICES; k++) {
+            DevCache &C = caches[(at + k) % CACHE_DEVICES];
+            std::vector<void *> out;
+            {
+                std::lock_guard<std::mutex> lk(C.mu);
+                if (!C.give(p)) continue;
+                while (C.held > CACHE_MAX) {
+                    void *s = C.evict();
+                    if (!s) break;                // what is left is in slabs that are in use
+                    out.push_back(s);
+                }
             }
+            for (void *s : out) mem.put(s);
+            return;
         }
-        for (void *s : out) mem.put(s);
     }
 
     // memory that a plan may count on beside what the runtime has free: the

@@ -158,6 +158,25 @@ static void reusable() {
     }
 }
 
+// a block goes back to the device it is of, whichever is current
+static void two_devices() {
+    Cache B;
+    size_t got;
+    void *a = B.alloc(4 * GiB, &got);
+    B.mem.current = 1;
+    void *b = B.alloc(6 * GiB, &got);
+    B.release(a);
+    EXPECT(B.caches[0].held == 4 * GiB && B.caches[1].held == 0);
+    consistent(B, 0);
+    consistent(B, 1);
+    EXPECT(B.alloc(4 * GiB, &got) != a);
+    B.mem.current = 0;
+    B.release(b);
+    EXPECT(B.caches[1].held == 6 * GiB && B.alloc(4 * GiB, &got) == a);
+    consistent(B, 0);
+    consistent(B, 1);
+}
+
 // any order of requests and releases leaves the lists in agreement
 static void any_order() {
     Cache B;
@@ -186,6 +205,7 @@ int main(int argc, char **argv) {
         {"cut_join_evict", cut_join_evict},
         {"full_card", full_card},
         {"reusable", reusable},
+        {"two_devices", two_devices},
         {"any_order", any_order},
     };
     for (auto &c : checks)

@@ -20,7 +20,7 @@ def check(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("name", ["cut_join_evict", "full_card", "reusable", "any_order"])
+@pytest.mark.parametrize("name", ["cut_join_evict", "full_card", "reusable", "two_devices", "any_order"])
 def test_block_cache(check, name):
     r = subprocess.run([check, name], stdout=subprocess.PIPE, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
