@@ -129,7 +129,8 @@ typedef struct omc_run_opts {
     int group;              /* Dij: beamlets transported together (0 = as many as hbm_budget allows,
                                1 = one beamlet at a time, the reference's loop order) */
     int64_t hbm_budget;     /* device bytes a Dij run may use for its tallies (0 = half the free memory,
-                               at most 96 GiB); dose runs: a quarter of it bounds the batch tallies */
+                               at most 96 GiB); dose runs: a quarter of it bounds the batch tallies, and
+                               the automatic event_target is 16384 where its pools fit it as well */
     int voxel_walk;         /* event form: 1 = photons fly voxel by voxel as the reference's photon()
                                does; 0 = delta tracking with the phantom's majorant (same distribution) */
     int electron_turns;     /* event form: refills of electron_budget steps an electron may hold its lane

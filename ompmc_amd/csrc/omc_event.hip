@@ -118,6 +118,10 @@ template <class R> size_t event_bytes(long long target) {
 // and 523 ms, the larger pools leaving less memory for tallies).  With photon
 // splitting a history carries nsplit times more electrons: 16384 in any case
 // (nsplit 20 on every 20th beamlet at 1, 2, 4 and 8 M: 1.40, 1.13, 1.05, 1.04 s).
+// The larger pools (12.9 GB in FP32, 17.2 GB in FP64, against 3.2 and 4.3) are
+// asked for only where the memory budget holds them beside the run's tallies,
+// and a run whose memory is taken by others meanwhile goes on with the smaller
+// ones (EvState::smaller).
 long long default_target(int dev, int nsplit, bool alone) {
     return (long long)device_cus(dev) * 4096 * (nsplit > 1 || alone ? 4 : 1);
 }
@@ -133,6 +137,7 @@ template <class R> struct EvState {
     Pool<R> pool[2][2];
     EvCtl *ctl = nullptr;
     long long target = 0, cap = 0, capmul = 8;   // pool capacity = capmul x target (peak in flight measured near 4x)
+    long long smaller = 0;                       // target to go on with where the pools do not fit (0: none)
     ~EvState() { A.release(); }
     int grow() {
         A.release();
@@ -140,6 +145,15 @@ template <class R> struct EvState {
         return alloc(target);
     }
     int alloc(long long tgt) {
+        int rc = try_alloc(tgt);
+        if (rc == OMC_ERR_NOMEM && smaller > 0 && smaller < tgt) {
+            A.release();
+            A.ok = true;
+            rc = try_alloc(smaller);
+        }
+        return rc;
+    }
+    int try_alloc(long long tgt) {
         target = tgt < 64 ? 64 : tgt;
         cap = capmul * target;
         // the charged pool's counter holds each band's length in 32 bits
@@ -327,9 +341,8 @@ size_t default_budget() {
 
 // Batches of a dose run transported in one job: o->batches_per_job, else as
 // many as a quarter of the memory budget holds tallies for.
-int batches_per_job(const omc_run_opts *o, int nbatch, size_t tally_bytes) {
+int batches_per_job(const omc_run_opts *o, int nbatch, size_t tally_bytes, size_t budget) {
     if (o->batches_per_job > 0) return std::min(o->batches_per_job, nbatch);
-    size_t budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : default_budget();
     size_t n = budget / 4 / std::max<size_t>(tally_bytes, 1);
     return (int)std::max<size_t>(1, std::min<size_t>(n, (size_t)nbatch));
 }
@@ -475,29 +488,34 @@ int omc_run_dosxyz_event(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const o
     // region array (slot = batch) and the batch statistics are taken in batch
     // order afterwards, so the result is the batch-by-batch one while the
     // job drains its longest tracks once instead of once per batch.
-    const int nbj = batches_per_job(o, nbatch, (size_t)nreg * sizeof(double));
-    long long tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit, true);
-    if (tgt > 4 * (long long)nper * nbj) tgt = std::max<long long>(4 * (long long)nper * nbj, 64);
-    int rc = S.alloc(tgt);
-    if (rc && o->event_target <= 0 && tgt > default_target(c->device, o->nsplit, false)) {
-        S.A.release();               // little memory left: the smaller pools
-        S.A.ok = true;
-        rc = S.alloc(default_target(c->device, o->nsplit, false));
+    const size_t half = default_budget(), budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : half;
+    const int nbj = batches_per_job(o, nbatch, (size_t)nreg * sizeof(double), budget);
+    const long long most = std::max<long long>(4 * (long long)nper * nbj, 64);     // a small job needs no more
+    long long tgt = std::min((long long)o->event_target, most);
+    if (tgt <= 0) {
+        tgt = std::min(default_target(c->device, o->nsplit, true), most);
+        S.smaller = std::min(default_target(c->device, o->nsplit, false), most);
+        const size_t need = event_bytes<R>(tgt) + (size_t)(nbj + 2) * nreg * sizeof(double);
+        if (need > std::min(budget, half)) tgt = S.smaller;
     }
-    if (rc) return rc;
+    // everything else the run needs comes before its pools, which can do with less
     double *d_e = A.alloc_n<double>((size_t)nbj * nreg), *d_s = A.alloc_n<double>(nreg),
            *d_s2 = A.alloc_n<double>(nreg);
     long *d_soff = A.alloc_n<long>(nbj + 1);
     unsigned long long *d_cnt = A.alloc_n<unsigned long long>(16);
     double *d_ebal = A.alloc_n<double>(2 * EB_N);
+    SrcDosxyz<R> dos;
+    int rc = make_dosxyz_src<R>(A, pd, src, dos);
+    if (rc) return rc;
     if (!A.ok) return omc_seterr(OMC_ERR_NOMEM, "device allocation failed");
+    rc = S.alloc(tgt);
+    if (rc) return rc;
     std::vector<long> soff(nbj + 1);
     for (int k = 0; k <= nbj; k++) soff[k] = (long)k * nper;
     CK(hipMemcpy(d_soff, soff.data(), sizeof(long) * (nbj + 1), hipMemcpyHostToDevice));
     EvLaunch<R> L;
     fill_launch(c, pd, S, o, L);
-    rc = make_dosxyz_src<R>(A, pd, src, L.src.dos);
-    if (rc) return rc;
+    L.src.dos = dos;
     L.src.use_beamlets = 0;
     L.src.slot_off = d_soff;
     L.endep = d_e;
@@ -711,7 +729,7 @@ template <class R> struct DijRun {
     long nreg, nvox, ntile;
     bool event, count, timing, replay, want_var, on_device, fused;
     double rel;
-    long long tgt;
+    long long tgt, smaller = 0;        // particles in flight; where their pools do not fit (EvState::smaller)
     std::vector<long> nper, gfirst;
     SrcBeamlets<R> bsrc;
     double *d_carry, *d_tdose, *d_tvar;
@@ -765,6 +783,7 @@ template <class R> int dij_lane_init(DijRun<R> &D, DijLane<R> &l) {
         }
         long long tgt = D.tgt;
         if (tgt > 4 * maxjob) tgt = std::max<long long>(4 * maxjob, 64);
+        l.S.smaller = D.smaller;
         int rc = l.S.alloc(tgt);
         if (rc) return rc;
         fill_launch(D.c, D.pd, l.S, o, l.L);
@@ -1059,7 +1078,11 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
         // one stream: the larger pools where they leave the plan as it is
         const long long big = default_target(c->device, o->nsplit, true);
         DijPlan p;
-        if (dij_plan(o, nreg, nbix, nbatch, big, budget, p) <= budget && p.G == plan.G && p.nbj == plan.nbj) D.tgt = big;
+        if (dij_plan(o, nreg, nbix, nbatch, big, budget, p) <= std::min(budget, default_budget()) && p.G == plan.G &&
+            p.nbj == plan.nbj) {
+            D.smaller = D.tgt;
+            D.tgt = big;
+        }
     }
     D.G = plan.G;
     D.NBJ = plan.nbj;
