@@ -81,13 +81,17 @@ constexpr int PHOTON_BLOCKS_PER_CU = OMC_PHOTON_BLOCKS_PER_CU;
 // SIMD of the charged kernel, three of the photon kernels.
 constexpr int CHARGED_WAVES_PER_CU = 8;
 constexpr int PHOTON_WAVES_PER_CU = 12;
-// LDS a charged-kernel workgroup may give to the electron bins (12 KB per
-// medium at 150 bins; two workgroups share a CU's 160 KB).  Plans with more
-// media read them from device memory.
+// LDS of a charged-kernel workgroup: two share a CU's 160 KB.
+constexpr size_t MAX_LDS_PER_GROUP = 80 * 1024;
+// LDS it may give to the electron bins (12 KB per medium at 150 bins).  Plans
+// with more media read them from device memory, and so do those whose bins do
+// not fit beside the planes (five media and 4700 planes): with 5432 planes 1e6
+// photon histories took 171 ms with the planes staged, 178 with the bins and 253
+// with both and one workgroup a CU (1e5 electrons of 9 MeV 164, 170, 256).
 constexpr size_t MAX_LDS_TABLES = 64 * 1024;
 // LDS it may give to the media's constants and the voxel planes: 4.2 KB on a
 // 256x256x200 phantom in FP32, 9 KB in FP64.  Phantoms with more planes than
-// this (about 5800 in FP32) read every table from device memory.
+// this (about 6000 in FP32, 3000 in FP64) read both from device memory.
 constexpr size_t MAX_LDS_GEOM = 24 * 1024;
 // Entries of a charged-kernel lane's deposit list (TallyList), 16 bytes each
 // for the 256 lanes of a workgroup; the lists are used where bins and lists
@@ -96,7 +100,6 @@ constexpr size_t MAX_LDS_GEOM = 24 * 1024;
 // three runs each).
 constexpr int TALLY_LIST = 6;
 constexpr size_t TALLY_LIST_BYTES = (size_t)TALLY_LIST * 256 * 16;
-constexpr size_t MAX_LDS_PER_GROUP = 80 * 1024;
 // Round guard of a job: the rounds its injection needs plus 2^16 -- with the
 // requeue after DEFAULT_TURNS x DEFAULT_BUDGET steps that is ~1.9e7 steps for
 // one particle, thousands of times the longest physical track.  A job that
@@ -372,18 +375,19 @@ template <class R> void fill_launch(omc_ctx *c, const PhantomDev *pd, EvState<R>
         const bool fp32 = std::is_same<R, float>::value;
         L.ebin = ht.cbin;
         const size_t bins = (size_t)ht.nmed * ht.cb_stride * sizeof(CBin<R>);
-        const bool stage_bins = fp32 && o->lds_tables >= 0 && bins <= MAX_LDS_TABLES;
-        L.lds_split = lds_layout<R>(ht.nmed, ph.nx, ph.ny, ph.nz, 0, 0);
-        if (L.lds_split.bytes <= (int)MAX_LDS_GEOM) {
-            L.st_split = ST_GEOM;
-            L.st_charged = stage_bins ? ST_GEOM | ST_BINS : ST_GEOM;
-            L.eb_words = stage_bins ? (int)(bins / 16) : 0;
+        auto layout = [&](int st, size_t list) {
+            return lds_layout<R>(st, ht.nmed, ph.nx, ph.ny, ph.nz, bins, list);
+        };
+        auto fits = [&](int st, size_t list) { return (size_t)layout(st, list).bytes <= MAX_LDS_PER_GROUP; };
+        if (layout(ST_GEOM, 0).bytes <= (int)MAX_LDS_GEOM) L.st_split = L.st_charged = ST_GEOM;
+        if (fp32 && o->lds_tables >= 0 && bins <= MAX_LDS_TABLES && fits(L.st_charged | ST_BINS, 0)) {
+            L.st_charged |= ST_BINS;
+            L.eb_words = (int)(bins / 16);
         }
-        // FP32: the deposit lists, where they fit beside the tables in two workgroups per CU
-        const size_t tables = L.st_charged ? (size_t)L.eb_words * 16 + L.lds_split.bytes : 0;
-        if (fp32 && tables + TALLY_LIST_BYTES <= MAX_LDS_PER_GROUP) L.tlist = TALLY_LIST;
-        L.lds_charged = lds_layout<R>(ht.nmed, ph.nx, ph.ny, ph.nz, (size_t)L.eb_words * 16,
-                                      L.tlist ? TALLY_LIST_BYTES : 0);
+        // FP32: the deposit lists, where they fit beside the tables
+        if (fp32 && fits(L.st_charged, TALLY_LIST_BYTES)) L.tlist = TALLY_LIST;
+        L.lds_split = layout(L.st_split, 0);
+        L.lds_charged = layout(L.st_charged, L.tlist ? TALLY_LIST_BYTES : 0);
     }
     int cus = device_cus(c->device);
     L.grid_event = o->grid > 0 ? o->grid : cus * PHOTON_BLOCKS_PER_CU;

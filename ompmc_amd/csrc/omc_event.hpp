@@ -115,17 +115,19 @@ __device__ __forceinline__ void note_drop(EvCtl *c, int why, int site, const Par
     }
 }
 
-// Dynamic LDS of an event kernel, byte offsets: the electron bins (ST_BINS)
-// from 0, then the media, their cut-offs and the voxel planes (ST_GEOM), then
-// the deposit lists (TallyList).  `bytes` is the whole.
+// Dynamic LDS of an event kernel that stages the tables of st, byte offsets: the
+// electron bins (ST_BINS) from 0, then the media, their cut-offs and the voxel
+// planes (ST_GEOM), then the deposit lists (TallyList).  `bytes` is the whole.
 struct LdsLayout { int med, ecut, planes, list, bytes; };
-template <class R> inline LdsLayout lds_layout(int nmed, int nx, int ny, int nz, size_t bin_bytes, size_t list_bytes) {
+template <class R>
+inline LdsLayout lds_layout(int st, int nmed, int nx, int ny, int nz, size_t bin_bytes, size_t list_bytes) {
     auto up = [](size_t n) { return (n + 15) / 16 * 16; };
+    const size_t geom = (st & ST_GEOM) != 0;
     LdsLayout l;
-    l.med = (int)up(bin_bytes);
-    l.ecut = l.med + (int)up(sizeof(Med<R>) * nmed);
-    l.planes = l.ecut + (int)up(sizeof(R) * MXMED);
-    l.list = l.planes + (int)up(sizeof(R) * (nx + ny + nz + 3));
+    l.med = (st & ST_BINS) != 0 ? (int)up(bin_bytes) : 0;
+    l.ecut = l.med + (int)(geom * up(sizeof(Med<R>) * nmed));
+    l.planes = l.ecut + (int)(geom * up(sizeof(R) * MXMED));
+    l.list = l.planes + (int)(geom * up(sizeof(R) * ((size_t)nx + ny + nz + 3)));
     l.bytes = l.list + (int)list_bytes;
     return l;
 }

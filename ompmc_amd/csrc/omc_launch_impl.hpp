@@ -80,7 +80,9 @@ template <class R> const void *event_kernel(int part, bool split, bool count, in
     if (count) return OMC_FN(k_event<R, false, true, 0>);
     // FP64 bins are not staged (twice the size, and the kernel has no room to gain from them)
     if constexpr (std::is_same<R, float>::value)
-        if (st & ST_BINS) return OMC_FN(k_event<R, false, false, ST_GEOM | ST_BINS>);
+        if (st & ST_BINS)
+            return st & ST_GEOM ? OMC_FN(k_event<R, false, false, ST_GEOM | ST_BINS>)
+                                : OMC_FN(k_event<R, false, false, ST_BINS>);
     return st ? OMC_FN(k_event<R, false, false, ST_GEOM>) : OMC_FN(k_event<R, false, false, 0>);
 #undef OMC_FN
 }
