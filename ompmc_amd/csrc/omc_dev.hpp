@@ -1883,7 +1883,8 @@ template <class R, class G, class T, int ST = 0> struct Engine {
     // remaining number of mean free paths and the cross section of the
     // fictitious method.  phase 0: enter electron() afresh; 1: resume;
     // 2: resume with the distance to the interaction still to be computed
-    // (after a step taken with a zero cross section).
+    // (after a step taken with a zero cross section); from 3: inside a vacuum,
+    // 4 + the medium before it (-1: none).
     struct EState { R demfp, sig0; int phase; };
 
     // condensed-history electron step (src/ompmc.c:4666-5451).  The variable
@@ -1898,8 +1899,9 @@ template <class R, class G, class T, int ST = 0> struct Engine {
 
     // The same routine, yielding after `budget` passes: returns 0 with the loop
     // state saved (es.phase 1 or 2 inside the reference's inner loop, 0 at the
-    // start of its outer loop, whose state is that of a fresh call); called
-    // again with that state it continues exactly where the uninterrupted
+    // start of its outer loop, whose state is that of a fresh call, and inside a
+    // vacuum that call and the medium before it, which the exit depends on);
+    // called again with that state it continues exactly where the uninterrupted
     // routine would.  Every other exit leaves es.phase = 0.
     //
     // The reference's two loops are one here, a step per pass.  Nearly every
@@ -1924,15 +1926,17 @@ template <class R, class G, class T, int ST = 0> struct Engine {
         R rhof_voxel = rhof;             // density of the current voxel, loaded with its medium at a move
         R eie = p.e;
         int iq = p.iq, qel = (1 + iq) / 2, medold = imed;
-        bool fresh = es.phase == 0;      // start of the reference's outer loop: a distance to the interaction is due
+        if (es.phase >= 3) medold = es.phase - 4;
+        // start of the reference's outer loop: a distance to the interaction is due
+        bool fresh = es.phase == 0 || es.phase >= 3;
         bool compute_tstep = es.phase != 1;
         if (fresh && eie <= ecut_of(imed)) return electron_stop(p, q, iq, eie, false);
         R eke = eie - RM, elke = (R)0, demfp = es.demfp, sig0 = es.sig0;
         int lelke = 0, iters = 0;
         es.phase = 0;
-        if (!fresh) {
+        if (!fresh || medold != imed) {
             elke = M<R>::log(eke);
-            lelke = pwlf_i(elke, med_of(imed).eke1, med_of(imed).eke0) - 1;
+            lelke = pwlf_i(elke, med_of(medold).eke1, med_of(medold).eke0) - 1;
         }
         for (;;) {
             R ustep = (R)0;
@@ -2171,12 +2175,17 @@ template <class R, class G, class T, int ST = 0> struct Engine {
                 lost += charged_energy(p);
                 return -1;
             }
-            // (never inside a vacuum: the medium before it is part of the state)
-            if (--budget <= 0 && imed != -1) {
-                es.demfp = demfp;
-                es.sig0 = sig0;
-                es.phase = fresh ? 0 : compute_tstep ? 2 : 1;
-                return 0;
+            if (--budget <= 0 && p.ix >= 0) {
+                // the energy bin is not part of the state: inside a vacuum it is
+                // the one of the medium before it, but for a particle that
+                // crossed another one there in a pass of length zero, which goes on
+                const bool in_vacuum = imed == -1 && medold != -1;
+                if (!in_vacuum || lelke == pwlf_i(elke, med_of(medold).eke1, med_of(medold).eke0) - 1) {
+                    es.demfp = demfp;
+                    es.sig0 = sig0;
+                    es.phase = in_vacuum ? 4 + medold : fresh ? 0 : compute_tstep ? 2 : 1;
+                    return 0;
+                }
             }
         }
         const CBin<R> cbi = bin(qel, imed, lelke);
