@@ -202,6 +202,12 @@ typedef struct omc_run_stats {
 
 /* Defaults: FP32, event form, keyed streams, seed 1802, nsplit 1, automatic launch. */
 void omc_run_opts_default(omc_run_opts *o);
+/* What the automatic settings (0) of the event form stand for on a device with
+ * photon splitting factor nsplit: event_target where a run has the device to
+ * itself (target[0]) and where streams or requests share it (target[1]),
+ * electron_budget, electron_turns and the most streams of a Dij run. */
+void omc_event_defaults(int device, int nsplit, int64_t target[2], int *electron_budget, int *electron_turns,
+                        int *streams);
 
 /* Dose run with omc_dosxyz semantics (main, omc_dosxyz.c:1206-1263):
  * nbatch batches of nperbatch histories; after each batch the per-region

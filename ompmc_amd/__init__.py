@@ -159,6 +159,8 @@ def lib():
     L.omc_phantom_upload.argtypes = [vp, C.POINTER(PhantomDesc), _i]
     L.omc_phantom_release.argtypes = [vp, C.c_int]
     L.omc_run_opts_default.argtypes = [C.POINTER(RunOpts)]
+    L.omc_event_defaults.argtypes = [C.c_int, C.c_int, _i64, _i, _i, _i]
+    L.omc_event_defaults.restype = None
     L.omc_run_dosxyz.argtypes = [vp, C.c_int, C.POINTER(DosxyzSourceDesc), C.c_int64, C.c_int,
                                  C.POINTER(RunOpts), _d, _d, C.POINTER(RunStats)]
     L.omc_run_dosxyz_noalloc.argtypes = [vp, C.c_int, C.POINTER(DosxyzSourceDesc), C.c_int64, C.c_int,
@@ -200,6 +202,16 @@ def _ip(a):
 def default_paths():
     return (os.path.join(DATA, "pegs4", "521icru.pegs4dat"), os.path.join(DATA, "pegs4", "pgs4form.dat"),
             DATA + "/")
+
+
+def event_defaults(device=0, nsplit=1):
+    """What the automatic settings of the event form stand for on a device:
+    event_target of a run that has it to itself and of streams that share it,
+    electron_budget, electron_turns and the most streams of a Dij run."""
+    t, v = (C.c_int64 * 2)(), [C.c_int() for _ in range(3)]
+    lib().omc_event_defaults(int(device), int(nsplit), t, *(C.byref(x) for x in v))
+    return dict(event_target_alone=t[0], event_target=t[1], electron_budget=v[0].value, electron_turns=v[1].value,
+                streams=v[2].value)
 
 
 def run_opts(precision=FP32, form=FORM_EVENT, seed=1802, rng=RNG_STREAMS, replay=None, replay_offsets=None,
@@ -317,6 +329,7 @@ class Context:
         _check(lib().omc_ctx_create(C.byref(h), len(media), arr, (pegs_file or pf).encode(),
                                     (pgs4form_file or ff).encode(), (data_folder or df).encode(), device))
         self.h = h
+        self.device = int(device)
         self.media = list(media)
 
     def close(self):

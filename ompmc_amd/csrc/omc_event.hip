@@ -129,6 +129,10 @@ long long default_target(int dev, int nsplit, bool alone) {
     return (long long)device_cus(dev) * 4096 * (nsplit > 1 || alone ? 4 : 1);
 }
 
+// Streams of a Dij run of several groups.  On the 1960-beamlet plan at 96 GiB:
+// 1 lane 7.2, 2 lanes 10.1, 3 lanes 10.4, 4 lanes 7-9 M histories/s.
+constexpr int DEFAULT_STREAMS = 3;
+
 // run_job's code for a pool overflow: the caller zeroes the job's tallies,
 // doubles the pools (EvState::grow) and runs the job again.  Every particle's
 // random stream is keyed by its history, so the rerun is the same job.
@@ -475,6 +479,15 @@ void stats_counters(omc_run_stats *st, const unsigned long long *cnt) {
 }
 
 }  // namespace
+
+extern "C" void omc_event_defaults(int device, int nsplit, int64_t target[2], int *electron_budget,
+                                   int *electron_turns, int *streams) {
+    target[0] = default_target(device, nsplit, true);
+    target[1] = default_target(device, nsplit, false);
+    *electron_budget = DEFAULT_BUDGET;
+    *electron_turns = DEFAULT_TURNS;
+    *streams = DEFAULT_STREAMS;
+}
 
 // ------------------------------------------------------------------ dose runs, event form
 template <class R>
@@ -1069,14 +1082,12 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
         if (n >= (1L << 32)) return omc_seterr(OMC_ERR_LIMIT, "more than 2^32 histories per batch of a beamlet");
     D.tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit, false);
     // lanes: up to three for an event-form run of several groups (o->streams
-    // pins the number), each planned on its share of the memory budget.  On
-    // the 1960-beamlet plan at 96 GiB: 1 lane 7.2, 2 lanes 10.1, 3 lanes
-    // 10.4, 4 lanes 7-9 M histories/s.
+    // pins the number), each planned on its share of the memory budget
     size_t budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : dij_default_budget();
     DijPlan plan;
     dij_plan(o, nreg, nbix, nbatch, D.tgt, budget, plan);
     int NL = 1;
-    if (D.event) NL = o->streams > 0 ? o->streams : std::min(3, (nbix + plan.G - 1) / plan.G);
+    if (D.event) NL = o->streams > 0 ? o->streams : std::min(DEFAULT_STREAMS, (nbix + plan.G - 1) / plan.G);
     if (NL > 1) dij_plan(o, nreg, nbix, nbatch, D.tgt, budget / NL, plan);
     if (NL == 1 && D.event && o->event_target <= 0) {
         // one stream: the larger pools where they leave the plan as it is
