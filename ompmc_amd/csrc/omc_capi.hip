@@ -206,21 +206,8 @@ template <class R> static int upload_tables(omc_ctx *c, DevArena &A, Tables<R> &
     T.ray_b = vec(h.ray_b, OMC_MXRAYFF);
     T.ray_c = vec(h.ray_c, OMC_MXRAYFF);
     T.ray_iarr = A.upload(std::vector<int>(h.ray_iarr, h.ray_iarr + OMC_RAYCDFSIZE));
-    T.esig = pw(h.esig0, h.esig1, nek);
-    T.psig = pw(h.psig0, h.psig1, nek);
-    T.ededx = pw(h.ededx0, h.ededx1, nek);
-    T.pdedx = pw(h.pdedx0, h.pdedx1, nek);
-    T.ebr1 = pw(h.ebr10, h.ebr11, nek);
-    T.pbr1 = pw(h.pbr10, h.pbr11, nek);
-    T.pbr2 = pw(h.pbr20, h.pbr21, nek);
-    T.tmxs = pw(h.tmxs0, h.tmxs1, nek);
-    T.blcce = pw(h.blcce0, h.blcce1, nek);
     T.etae = pw(h.etae_ms0, h.etae_ms1, nek);
     T.etap = pw(h.etap_ms0, h.etap_ms1, nek);
-    T.q1ce = pw(h.q1ce_ms0, h.q1ce_ms1, nek);
-    T.q1cp = pw(h.q1cp_ms0, h.q1cp_ms1, nek);
-    T.q2ce = pw(h.q2ce_ms0, h.q2ce_ms1, nek);
-    T.q2cp = pw(h.q2cp_ms0, h.q2cp_ms1, nek);
     T.range_ep = vec(h.range_ep, 2 * nek);
     T.e_array = vec(h.e_array, nek);
     T.spin_rej = vec(h.spin_rej, (size_t)nm * OMC_NSPIN_MED + 1);   // + the zero entry of quirk Q17

@@ -155,8 +155,10 @@ template <class R> __device__ __forceinline__ PW<R> gld(const PW<R> *p) {
 // multiple scattering and its discrete interaction read at the particle's
 // own bin, so a step touches one or two cache lines instead of eight tables.
 // Tables::cbin holds them as [2][nmed][cb_stride] (electrons, positrons;
-// cb_stride = the largest MEKE + 1); the per-quantity arrays stay for reads
-// at other bins (the range walk of eloss, the end of a step's interval).
+// cb_stride = the largest MEKE + 1).  Kernels without staged bins read what they
+// need of other bins from arrays of one quantity: etae and etap at the end of a
+// step, range_ep and e_array in the range walk of eloss and at the interaction
+// site's bin.
 // The fields of a step come first, those of one 16-byte read side by side.
 template <class R> struct alignas(16) CBin {
     R e_lo, range;                                          // e_array and range_ep at the bin
@@ -181,8 +183,7 @@ template <class R> struct Tables {
     const PW<R> *gmfp, *gbr1, *gbr2, *cohe, *pmax;              // [nmed*MXGE]
     const R *ray_xgrid, *ray_fcum, *ray_b, *ray_c;              // medium 0 only (reference quirk Q1)
     const int *ray_iarr;
-    const PW<R> *esig, *psig, *ededx, *pdedx, *ebr1, *pbr1, *pbr2, *tmxs;
-    const PW<R> *blcce, *etae, *etap, *q1ce, *q1cp, *q2ce, *q2cp; // [nmed*MXEKE]
+    const PW<R> *etae, *etap;                                   // [nmed*MXEKE]
     const R *range_ep;                                          // [2][nmed][MXEKE]
     const R *e_array;                                           // [nmed][MXEKE]
     const R *spin_rej;                                          // [nmed][NSPIN_MED]
