@@ -349,6 +349,7 @@ size_t default_budget() {
 // Batches of a dose run transported in one job: o->batches_per_job, else as
 // many as a quarter of the memory budget holds tallies for.
 int batches_per_job(const omc_run_opts *o, int nbatch, size_t tally_bytes, size_t budget) {
+    nbatch = std::min(nbatch, MAX_SLOTS);
     if (o->batches_per_job > 0) return std::min(o->batches_per_job, nbatch);
     size_t n = budget / 4 / std::max<size_t>(tally_bytes, 1);
     return (int)std::max<size_t>(1, std::min<size_t>(n, (size_t)nbatch));
@@ -646,8 +647,8 @@ size_t dij_plan(const omc_run_opts *o, long nreg, int nbix, int nbatch, long lon
     const size_t room = budget > fixed ? budget - fixed : 0;
     const int gmax = std::min(nbix, 4096);
     long best_jobs = -1;
-    int lo = 1, hi = nbatch;
-    if (o->batches_per_job > 0) lo = hi = std::min(o->batches_per_job, nbatch);
+    int lo = 1, hi = std::min(nbatch, MAX_SLOTS / std::max(gmax, 1));
+    if (o->batches_per_job > 0) lo = hi = std::min(o->batches_per_job, hi);
     for (int nbj = hi; nbj >= lo; nbj--) {
         long g = o->group > 0 ? std::min(o->group, nbix) : (long)(room / dij_slot_bytes(nreg, nbj));
         g = std::max(1L, std::min<long>(g, gmax));

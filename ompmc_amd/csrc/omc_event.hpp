@@ -172,7 +172,8 @@ __device__ __forceinline__ uint4 pack2(double a, double b) {
 __device__ __forceinline__ double lo2(const uint4 &v) { return __hiloint2double((int)v.y, (int)v.x); }
 __device__ __forceinline__ double hi2(const uint4 &v) { return __hiloint2double((int)v.w, (int)v.z); }
 
-// the slot word carries the charge as well (slot counts stay far below 2^29)
+// the slot word carries the charge as well, which leaves the slot 30 bits
+constexpr int MAX_SLOTS = 1 << 30;
 __device__ __forceinline__ uint32_t slot_word(int slot, int iq) { return ((uint32_t)slot << 2) | (uint32_t)(iq + 1); }
 
 __device__ __forceinline__ void load(const Pool<float> &P, long long i, Queued<float> &q) {
