@@ -62,11 +62,11 @@ template <> struct M<double> {
     static __device__ __forceinline__ double fmax(double a, double b) { return ::fmax(a, b); }
     static __device__ __forceinline__ double fmin(double a, double b) { return ::fmin(a, b); }
     static __device__ __forceinline__ double fabs(double a) { return ::fabs(a); }
-    // x^3 and x^4 through pow(): repeated products round differently in a
-    // large share of cases, and the FP64 path must round as the reference does
     // a * b + c as each path rounds it: in one rounding in float (where the
     // compiler contracts such expressions within a block anyway), in two in double
     static __device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
+    // x^3 and x^4 through pow(): repeated products round differently in a
+    // large share of cases, and the FP64 path must round as the reference does
     static __device__ __forceinline__ double pow3(double x) { return ::pow(x, 3.0); }
     static __device__ __forceinline__ double pow4(double x) { return ::pow(x, 4.0); }
     // remaining path (cm at the medium's nominal density) below which an
@@ -1917,7 +1917,7 @@ template <class R, class G, class T, int ST = 0> struct Engine {
     // a value outside its physical range).  With half of a wave's lanes in
     // zero-length passes, every pass paid for all branches of a step: folded,
     // 1e4 histories on 32^3 water 7.5 -> 6.0 ms, 2e5 9 MeV electrons on a CT
-    // 79.5 -> 65 ms, 1e7 histories on the 128^3 slab 427 -> 389 ms (194 passes a
+    // 79.5 -> 66 ms, 1e7 histories on the 128^3 slab 427 -> 382 ms (194 passes a
     // history before).
     __device__ __forceinline__ int electron_run(Part<R> &p, Part<R> &q, EState &es, int budget) {
         const R RM = (R)0.5109989461;

@@ -66,9 +66,11 @@ int device_cus(int dev) {
 // whose particles have ended; a refill costs one atomic's and a few loads' wait.
 constexpr int DEFAULT_BUDGET = 4;
 constexpr int DEFAULT_TURNS = 30;
-// Workgroups per compute unit of the persistent event kernels.  Whole c3
-// plan, best of three (M histories/s), charged x photon: 8 x 8 21.9,
-// 2 x 8 22.0, 2 x 4 22.2, 4 x 4 21.9 -- within run-to-run noise.
+// Workgroups per compute unit of the persistent event kernels.  The registers
+// hold two of the charged kernel at once; launched with 8, 4 and 2, 3e6
+// histories on the 128^3 slab took 62.3, 60.7 and 61.8 ms, 2e5 electrons of 9 MeV
+// on a CT 57.9, 58.2 and 58.3, 1e4 histories on 32^3 water 5.8 each: the same to
+// run-to-run noise.
 #ifndef OMC_CHARGED_BLOCKS_PER_CU
 #define OMC_CHARGED_BLOCKS_PER_CU 8
 #endif
@@ -94,15 +96,15 @@ constexpr size_t MAX_LDS_TABLES = 64 * 1024;
 // this (about 6000 in FP32, 3000 in FP64) read both from device memory.
 constexpr size_t MAX_LDS_GEOM = 24 * 1024;
 // Entries of a charged-kernel lane's deposit list (TallyList), 16 bytes each
-// for the 256 lanes of a workgroup; the lists are used where bins and lists
-// together leave room for two workgroups per CU.  Eight entries measured the
+// for the 256 lanes of a workgroup; the lists are used where they fit beside
+// the tables.  Eight entries measured the
 // same as six on the 1960-beamlet plan (22.55 against 22.64 M histories/s,
 // three runs each).
 constexpr int TALLY_LIST = 6;
 constexpr size_t TALLY_LIST_BYTES = (size_t)TALLY_LIST * 256 * 16;
 // Round guard of a job: the rounds its injection needs plus 2^16 -- with the
-// requeue after DEFAULT_TURNS x DEFAULT_BUDGET steps that is ~1.9e7 steps for
-// one particle, thousands of times the longest physical track.  A job that
+// requeue after DEFAULT_TURNS x DEFAULT_BUDGET steps that is 7.9e6 steps for
+// one particle, hundreds of times the longest tracks seen.  A job that
 // has not drained by then is reported as a step-guard error.
 long max_rounds(long long nhist, long long target) { return 65536L + 8L * (long)(nhist / std::max(target, 1LL)); }
 

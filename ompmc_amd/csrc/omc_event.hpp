@@ -437,14 +437,15 @@ __device__ __forceinline__ void flush_counters(unsigned long long *dst, const Co
 // condensed-history steps of electron_run() -- then the wave meets: lanes
 // whose particle left, or turned into the other type, hand it and any
 // secondary to the output queues and claim the next queued particle (one
-// atomic per wave).  A particle of this kernel's type stays in its lane until
+// atomic instruction a trip, wave_exchange).  A particle of this kernel's type stays in its lane until
 // it is gone, so the queues only carry new secondaries and type changes, and
 // no lane idles while the queue still holds work.  The wave exits when its
 // lanes are empty and the queue is exhausted.
 //
-// Two things keep a launch short.  A wave reads the claim counter before it
-// bumps it, so once the queue is exhausted idle waves leave without
-// serialising on that one address (8192 waves queueing on it cost ~100 us
+// Two things keep a launch short.  A wave reads the claim counter before its
+// first claim, and claims no more once a claim has come back from beyond the
+// queue's end, so idle waves of an exhausted queue leave without serialising on
+// that one address (8192 waves queueing on it cost ~100 us
 // per launch).  And an electron that has held its lane for a.turns refills
 // is handed back to the queue with its resumable state (position in its
 // random stream, distance to the next discrete interaction, step phase): an

@@ -224,17 +224,17 @@ template <> __device__ __forceinline__ void make_rng<double, Replay>(Replay &g, 
     g.err = a.err + 1;
 }
 
-// Lanes of a wavefront that take particles (histories): all 64 where the queue fills the
-// wavefronts the device holds at once, else an even share of the queue.  A
+// Lanes of a wavefront that take particles (histories): all 64 where the queue
+// fills the wavefronts the device holds at once, else an even share of it.  A
 // pass of a wave's loop runs every branch any of its lanes takes, and its
 // rejection and voxel loops as long as the slowest lane, so the few particles
 // of a small job, or of the last rounds of any job, finish sooner one or a few
 // to a wave on many SIMDs than 64 to a wave on a few of them.  Which lane holds
 // a particle does not change its track.  Measured: 1e4 histories on 32^3
-// water 9.5 -> 8.5 ms, 2e5 9 MeV electrons on a CT 98 -> 91 ms, a 21-beamlet
-// matrix 21.2 -> 18.5 ms, 1e5 histories at nsplit 20 on a CT 127 -> 105 ms, 1e7
-// histories on the 128^3 slab the same to 1%; with
-// half or twice the wavefronts (1024, 4096) the same to 5%.  In the history
+// water 9.5 -> 8.3 ms, 2e5 9 MeV electrons on a CT 98 -> 91 ms, a 21-beamlet
+// matrix 21.3 -> 18.5 ms, 1e5 histories at nsplit 20 on a CT 127 -> 105 ms, 1e7
+// histories on the 128^3 slab the same to 1%; with half or twice the
+// wavefronts (1024, 4096) the same to 5%.  In the history
 // form, whose lanes run whole showers: 1e5 histories in batches of 1e4 on a 64^3
 // slab 430 -> 169 ms.  waves 0: always 64.
 __device__ __forceinline__ int lane_share(long long n, int waves) {

@@ -78,7 +78,9 @@ template <class R> const void *event_kernel(int part, bool split, bool count, in
                      : st ? OMC_FN(k_event_split<R, false, ST_GEOM>) : OMC_FN(k_event_split<R, false, 0>);
     if (part == 1) return count ? OMC_FN(k_event<R, true, true, 0>) : OMC_FN(k_event<R, true, false, 0>);
     if (count) return OMC_FN(k_event<R, false, true, 0>);
-    // FP64 bins are not staged (twice the size, and the kernel has no room to gain from them)
+    // FP64 bins (24 KB a medium) are read from device memory.  Staged in a trial,
+    // 1e6 histories on 60^3 water took 36.3 ms against 39.6; with four media they
+    // do not fit beside a second workgroup.
     if constexpr (std::is_same<R, float>::value)
         if (st & ST_BINS)
             return st & ST_GEOM ? OMC_FN(k_event<R, false, false, ST_GEOM | ST_BINS>)
