@@ -60,6 +60,12 @@ std::vector<void *> pinned_free;
 
 }  // namespace
 
+void *device_alloc(size_t n) {
+    HipMem &mem = dev_blocks().mem;
+    if (void *p = mem.get(n)) return p;
+    devcache_trim();
+    return mem.get(n);
+}
 void *devcache_alloc(size_t n, size_t *got) { return dev_blocks().alloc(n, got); }
 void devcache_free(void *p, size_t) { dev_blocks().release(p); }
 size_t devcache_reusable() { return dev_blocks().reusable(); }
@@ -152,8 +158,7 @@ void *DevArena::alloc(size_t n) {
     if (cached) {
         p = devcache_alloc(got, &got);
         if (!p) return nullptr;
-    } else if (hipMalloc(&p, got) != hipSuccess) {
-        (void)hipGetLastError();
+    } else if (!(p = device_alloc(got))) {
         return nullptr;
     }
     blocks.emplace_back(p, got);

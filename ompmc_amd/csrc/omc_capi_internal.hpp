@@ -49,6 +49,8 @@ struct DevArena {
 // returns to the runtime all of it that shares no allocation with a block in
 // use.
 void *devcache_alloc(size_t n, size_t *got);
+// an allocation of the runtime, for which the cache gives way
+void *device_alloc(size_t n);
 void devcache_free(void *p, size_t n);
 size_t devcache_reusable();
 void devcache_trim();

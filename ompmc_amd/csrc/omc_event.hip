@@ -1209,9 +1209,8 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
         int64_t *d_ir = nullptr;
         double *d_val = nullptr;
         if (D.on_device) {
-            if (hipMalloc(&d_ir, sizeof(int64_t) * (nnz ? nnz : 1)) != hipSuccess) d_ir = nullptr;
-            if (hipMalloc(&d_val, sizeof(double) * (nnz ? nnz : 1)) != hipSuccess) d_val = nullptr;
-            (void)hipGetLastError();
+            d_ir = (int64_t *)device_alloc(sizeof(int64_t) * (nnz ? nnz : 1));
+            d_val = (double *)device_alloc(sizeof(double) * (nnz ? nnz : 1));
         } else {
             d_ir = T.alloc_n<int64_t>((size_t)(nnz ? nnz : 1));
             d_val = T.alloc_n<double>((size_t)(nnz ? nnz : 1));

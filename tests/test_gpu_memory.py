@@ -1,4 +1,4 @@
-"""Dose runs where little device memory is free.  A run alone on its stream keeps
+"""Dose runs and phantoms where little device memory is free.  A run alone on its stream keeps
 more particles in flight, in pools of 12.9 GB (FP32) or 17.2 GB (FP64), where
 the memory holds them beside its batch tallies; where it does not, the run goes
 through with smaller pools, and gives the same dose up to the order of its FP64
@@ -57,3 +57,19 @@ def test_dose_run_with_little_free_memory(precision, entry, beside):
     for x in (got, again):
         for a, b in zip(x, ref):
             assert np.allclose(a, b, rtol=1e-10, atol=1e-12 * b.max())
+
+
+def test_phantom_where_the_rest_is_kept_for_runs():
+    """A phantom goes into memory that the library only keeps for later runs."""
+    ph = P.water_cube(220, 0.1)                          # 310 MB on the device
+    c = omc.Context(ph.media)
+    small = c.phantom(P.water_cube(20, 0.5))
+    c.run_dosxyz(small, omc.Spectrum.mono(2.0), 110_000, 10, collimator=(-1, 1, -1, 1),
+                 event_target=torch.cuda.get_device_properties(0).multi_processor_count * 4096)
+    fill = _leave(200 << 20)                             # 3.2 GB are kept
+    try:
+        c.phantom(ph).release()
+    finally:
+        del fill
+        torch.cuda.empty_cache()
+        c.close()
