@@ -508,7 +508,10 @@ int omc_run_dosxyz_event(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const o
     // region array (slot = batch) and the batch statistics are taken in batch
     // order afterwards, so the result is the batch-by-batch one while the
     // job drains its longest tracks once instead of once per batch.
-    const size_t half = default_budget(), budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : half;
+    // (a server's requests name both: asking the runtime for the free memory takes
+    // some 30 us, and every request's thread would)
+    const size_t half = o->batches_per_job > 0 && o->event_target > 0 ? 0 : default_budget();
+    const size_t budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : half;
     const int nbj = batches_per_job(o, nbatch, (size_t)nreg * sizeof(double), budget);
     const long long most = std::max<long long>(4 * (long long)nper * nbj, 64);     // a small job needs no more
     long long tgt = std::min((long long)o->event_target, most);
@@ -641,10 +644,10 @@ struct DijPlan {
 // at most 96 GiB.  Past ~100 GiB held by the process, allocations cost
 // seconds to map and unmap (measured on the 1960-beamlet plan: 128-144 GiB
 // runs lost 2-5 s per call, 96 GiB none) while saving only a few jobs.
-size_t dij_default_budget() { return std::min(default_budget(), (size_t)96 << 30); }
+constexpr size_t MAX_DIJ_BUDGET = (size_t)96 << 30;
 
 size_t dij_plan(const omc_run_opts *o, long nreg, int nbix, int nbatch, long long target, size_t budget, DijPlan &P) {
-    if (!budget) budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : dij_default_budget();
+    if (!budget) budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : std::min(default_budget(), MAX_DIJ_BUDGET);
     const size_t fixed = dij_fixed_bytes(nreg, o, target);
     const size_t room = budget > fixed ? budget - fixed : 0;
     const int gmax = std::min(nbix, 4096);
@@ -1086,17 +1089,18 @@ int run_dij(omc_ctx *c, hipStream_t stream, PhantomDev *pd, const omc_spectrum_d
     D.tgt = o->event_target > 0 ? o->event_target : default_target(c->device, o->nsplit, false);
     // lanes: up to three for an event-form run of several groups (o->streams
     // pins the number), each planned on its share of the memory budget
-    size_t budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : dij_default_budget();
+    const size_t half = default_budget();
+    const size_t budget = o->hbm_budget > 0 ? (size_t)o->hbm_budget : std::min(half, MAX_DIJ_BUDGET);
     DijPlan plan;
     dij_plan(o, nreg, nbix, nbatch, D.tgt, budget, plan);
     int NL = 1;
     if (D.event) NL = o->streams > 0 ? o->streams : std::min(DEFAULT_STREAMS, (nbix + plan.G - 1) / plan.G);
     if (NL > 1) dij_plan(o, nreg, nbix, nbatch, D.tgt, budget / NL, plan);
-    if (NL == 1 && D.event && o->event_target <= 0) {
+    if (NL == 1 && D.event && !given && o->event_target <= 0) {
         // one stream: the larger pools where they leave the plan as it is
         const long long big = default_target(c->device, o->nsplit, true);
         DijPlan p;
-        if (dij_plan(o, nreg, nbix, nbatch, big, budget, p) <= std::min(budget, default_budget()) && p.G == plan.G &&
+        if (dij_plan(o, nreg, nbix, nbatch, big, budget, p) <= std::min(budget, half) && p.G == plan.G &&
             p.nbj == plan.nbj) {
             D.smaller = D.tgt;
             D.tgt = big;
